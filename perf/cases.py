@@ -56,8 +56,9 @@ def listed():
         _search("plain session bcc16", "session", "BCC", 16, bcc5, 512, 256, iters=2),
         # 108000 sites, plain: one lattice a CU, neighbour table beyond an L2
         _search("plain session fcc30", "session", "FCC", 30, eq5, 256, 512),
-        # 500000 sites, plain: the species stay in HBM
-        _search("plain local search fcc50", "local", "FCC", 50, fcc6, 64, 256, depth=10),
+        # a population beyond LDS, plain: the species stay in HBM (256000 sites, of
+        # which a search of an unlucky target takes about a second)
+        _search("plain local search fcc40", "local", "FCC", 40, fcc6, 64, 256, depth=10),
         # the time-to-fitness workload: guided and batched, one problem
         _search("guided batch fcc30", "batch", "FCC", 30, eq5, 256, 512, cand=12, accepts=8),
         # guided at the example's size, where the rounds are short
@@ -90,7 +91,7 @@ def draw(rng):
                     task=rng.randint(64, 300), depth=rng.randint(4, 10), iters=1)
     latt = rng.choice(["FCC", "BCC"])
     edge = logint(4, 32 if latt == "FCC" else 40) if rng.random() < 0.9 else \
-        (rng.randint(33, 48) if latt == "FCC" else rng.randint(41, 60))
+        (rng.randint(33, 40) if latt == "FCC" else rng.randint(41, 50))
     n = _BASIS[latt] * edge ** 3
     k = rng.randint(2, 5 if what == "guided" else 8) if rng.random() < 0.3 else rng.randint(3, 5)
     species = " ".join(str(rng.randint(1, 6) * 5) for _ in range(k))
