@@ -22,6 +22,7 @@
 #include "../../include/pyhea_hcs.h"
 #include "hea_internal.h"
 #include "hea_sort.h"
+#include "hea_stencil.h"
 
 // Workspace of hea_local_mc_device_noalloc: the local search's iteration
 // word, per-lattice counters and pair counts live here instead of in
@@ -457,6 +458,7 @@ struct hea_problem_s {
   bool walk_gather = false;        // PYHEA_AMD_WALK_GATHER=1: no neighbour records in the walk
   int guide_blk = 4;               // guided candidates from blocks of 2^b sites (16; 0: uniform);
                                    // PYHEA_AMD_GUIDE_BLOCK=b sets b
+  int lt = HEA_LT_NONE, edge = 0;  // stencil lattice (hea_stencil.h): shell set, cells per axis
   int64_t max_lds = 0;
   DevBuf<HeaConst> d_const;
   DevBuf<int32_t> d_nbr;
@@ -652,6 +654,17 @@ void fill_problem_args(hea_problem p, HeaMcArgs& a) {
     a.weight[s] = c.weight[s];
   }
   a.g_blk = p->guide_blk;
+  a.lt = p->lt;
+  a.edge = p->edge;
+  a.inv_edge = p->edge > 0 ? 1.0f / (float)p->edge : 0.0f;
+  a.n_magic = (uint32_t)((1ull << 32) / (uint64_t)c.N);
+}
+
+// Launch of a plain search of `task` proposals a round by the stencil-lattice
+// kernel (threads = 0: the problem or round size is not for it).
+HeaSearchPlan search_plan(hea_problem p, int task) {
+  if (p->force_hbm_species) return HeaSearchPlan();
+  return hea_search_plan(p->hc, p->lt, task, p->max_lds);
 }
 
 int launch_mc(hea_problem p, uint8_t* lat, double* fit, const int32_t* counts, int64_t* stats,
@@ -660,8 +673,7 @@ int launch_mc(hea_problem p, uint8_t* lat, double* fit, const int32_t* counts, i
               hipStream_t st, const GuideCfg& gd = GuideCfg(), int tp = 0,
               unsigned long long* rec = nullptr) {
   HeaMcArgs a;
-  a.pc = p->d_const.p;
-  a.nbr = p->d_nbr.p;
+  fill_problem_args(p, a);
   a.lattices = lat;
   a.fitness = fit;
   a.counts = counts;
@@ -679,21 +691,18 @@ int launch_mc(hea_problem p, uint8_t* lat, double* fit, const int32_t* counts, i
   a.g_cand = gd.cand;
   a.g_tau = gd.tau;
   a.g_multi = gd.multi;
-  a.g_blk = p->guide_blk;
   a.dbg_pairs = gd.dbg_pairs;
   a.dbg_pred = gd.dbg_pred;
   a.rec = rec;
-  const HeaConst& c = p->hc;
-  a.N = c.N;
-  a.K = c.K;
-  a.S = c.S;
-  a.stride = c.stride;
-  for (int s = 0; s < HEA_MAX_S; ++s) {
-    a.Z[s] = c.Z[s];
-    a.off[s] = c.off[s];
-    a.delta[s] = c.delta[s];
-    a.weight[s] = c.weight[s];
+  if (!gd.hist) {
+    const HeaSearchPlan plan = search_plan(p, task);
+    if (plan.threads) {
+      a.dl = plan.dl;
+      HEA_HIP(hea_launch_search(a, plan, st));
+      return HEA_OK;
+    }
   }
+  const HeaConst& c = p->hc;
   a.dw = hea_mc_draw_lanes(task, c.conc, c.K, hea_mc_split(a, p->hc.self_nbr != 0));
   HEA_HIP(hea_launch_local_mc(a, p->hc.K, sp_lds, p->hc.self_nbr != 0, lds, st));
   return HEA_OK;
@@ -710,8 +719,8 @@ int check_run_args(hea_problem p, int L, int task, int depth) {
 
 // Whether the walk of a launch with this species placement uses neighbour
 // records: species read from HBM, records that fit one word, no override.
-bool use_records(hea_problem p, bool sp_lds) {
-  return !sp_lds && !p->walk_gather &&
+bool use_records(hea_problem p, bool sp_lds, int task) {
+  return !sp_lds && !search_plan(p, task).threads && !p->walk_gather &&
          hea_records_fit(p->hc.K, p->hc.S, p->hc.Z, p->hc.self_nbr != 0);
 }
 
@@ -728,6 +737,8 @@ int mc_lds(hea_problem p, int task, size_t* lds, bool* sp_lds, int tp = 0) {
     if ((int64_t)*lds > p->max_lds) return fail(HEA_EUNSUPPORTED, "parallel_task too large for LDS");
   }
   HEA_HIP(hea_prepare_local_mc(p->hc.K, *sp_lds, self, *lds));
+  if (search_plan(p, task).threads)
+    HEA_HIP(hea_prepare_search(p->lt, p->hc.K, (size_t)p->max_lds));
   return HEA_OK;
 }
 
@@ -765,9 +776,11 @@ int hea_problem_create(const hea_problem_desc* d, int device, hea_problem* out) 
   for (size_t e = 0; e < (size_t)N * sumZ; ++e)
     if (d->nbr[e] < 0 || d->nbr[e] >= N) return fail(HEA_EINVAL, "neighbour index out of range");
   // The neighbour relation must be symmetric with multiplicity so that the
-  // pair counts, and hence gamma, are symmetric.
-  int self = 0;
-  {
+  // pair counts, and hence gamma, are symmetric.  A table that is a lattice's
+  // stencil is: its shells hold every vector with its opposite, once.
+  int self = 0, edge = 0;
+  const int lt = hea_stencil_detect(d->nbr, N, S, d->shell_size, &edge);
+  if (lt == HEA_LT_NONE) {
     int o = 0;
     for (int s = 0; s < S; ++s) {
       const int z = d->shell_size[s];
@@ -796,6 +809,8 @@ int hea_problem_create(const hea_problem_desc* d, int device, hea_problem* out) 
 
   hea_problem p = new hea_problem_s();
   p->device = device;
+  p->lt = lt;
+  p->edge = edge;
   {
     const char* v = getenv("PYHEA_AMD_SPECIES_IN_HBM");
     p->force_hbm_species = v && v[0] == '1';
@@ -945,7 +960,7 @@ static int local_mc_enqueue(hea_problem p, int L, uint8_t* lat, double* fit, int
   int rc = mc_lds(p, task, &lds, &sp_lds);
   if (rc) return rc;
   unsigned long long* rec = nullptr;
-  if (records && use_records(p, sp_lds)) {
+  if (records && use_records(p, sp_lds, task)) {
     const size_t n = (size_t)L * p->hc.N;
     if (p->d_rec.n < n) HEA_HIP(p->d_rec.alloc(n));
     rec = p->d_rec.p;
@@ -1045,7 +1060,7 @@ int hea_local_mc_device_noalloc(hea_problem p, int32_t L, void* d_lattices, void
 // (the buffer is guided mode's records when guided, the same size).
 static int session_records(hea_session s) {
   s->rec = nullptr;
-  if (!use_records(s->p, s->sp_lds)) return HEA_OK;
+  if (!use_records(s->p, s->sp_lds, s->task)) return HEA_OK;
   const size_t n = (size_t)s->L * s->p->hc.N;
   if (s->hist.n < n) {
     HEA_HIP(s->hist.alloc(n));
@@ -1492,7 +1507,13 @@ static int batch_enqueue_iteration(hea_batch b, const IterHooks* hk = nullptr) {
                                hipMemcpyDeviceToDevice, st));
       HEA_HIP(hipEventRecord(hk->ev[2 * h], st));
     }
-    if (P == 1)  // one problem: nothing to balance, its arguments go in the kernarg segment
+    const HeaSearchPlan plan =
+        P == 1 && !b->guide.hist ? search_plan(b->probs[0], b->task) : HeaSearchPlan();
+    if (plan.threads) {
+      HeaMcArgs a = b->hmargs[h];
+      a.dl = plan.dl;
+      HEA_HIP(hea_launch_search(a, plan, st));
+    } else if (P == 1)  // nothing to balance: the arguments go in the kernarg segment
       HEA_HIP(hea_launch_local_mc(b->hmargs[h], b->probs[0]->hc.K, b->sp_lds, false, b->lds, st));
     else
       HEA_HIP(hea_launch_local_mc_batch(ba, b->kmax, b->sp_lds, b->guide.hist != nullptr, b->grid,
@@ -1671,6 +1692,8 @@ int hea_batch_create(const hea_problem* probs, int32_t n_probs, int32_t L, int32
   if (e == hipSuccess) e = hea_prepare_local_mc_batch(b->kmax, b->sp_lds, b->lds);
   if (e == hipSuccess && n_probs == 1)
     e = hea_prepare_local_mc(probs[0]->hc.K, b->sp_lds, false, b->lds);
+  if (e == hipSuccess && n_probs == 1 && search_plan(probs[0], task).threads)
+    e = hea_prepare_search(probs[0]->lt, probs[0]->hc.K, (size_t)probs[0]->max_lds);
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking);
   if (e != hipSuccess) {
     delete b;
@@ -1719,7 +1742,7 @@ static int batch_records(hea_batch b) {
   size_t n = 0;
   bool any = false;
   for (int q = 0; q < P; ++q) {
-    use[q] = use_records(b->probs[q], b->sp_lds);
+    use[q] = use_records(b->probs[q], b->sp_lds, b->task);
     any = any || use[q];
     off[q] = n;
     n += (size_t)b->L * b->probs[q]->hc.N;

@@ -79,6 +79,11 @@ struct HeaMcArgs {
   int32_t N, K, S, stride;
   int32_t Z[HEA_MAX_S], off[HEA_MAX_S];
   double delta[HEA_MAX_S], weight[HEA_MAX_S];
+  // stencil lattices (hea_stencil.h; lt = HEA_LT_NONE: any other table)
+  int32_t lt, edge;        // shell set and cells per axis
+  float inv_edge;          // 1 / edge (hea_cell_div_small)
+  uint32_t n_magic;        // floor(2^32 / N)
+  int32_t dl;              // k_search: draw lanes of two draws each
 };
 
 // One launch of the persistent local search over many problems: probs[p]
@@ -134,6 +139,16 @@ __device__ __forceinline__ double hea_r_of_count(const HeaConst& P, int s, int64
   while (q + 1 < P.nseg[s] && P.seg_k0[s][q + 1] <= k) ++q;
   return fma((double)(k - P.seg_k0[s][q]), P.seg_inc[s][q], P.seg_v0[s][q]);
 }
+
+// Launch of the stencil-lattice search (hea_search.hip); threads = 0: not for
+// this problem and round size.
+struct HeaSearchPlan {
+  int threads = 0, dl = 0;
+  size_t lds = 0;
+};
+HeaSearchPlan hea_search_plan(const HeaConst& c, int lt, int task, int64_t max_lds);
+hipError_t hea_prepare_search(int lt, int K, size_t lds);
+hipError_t hea_launch_search(const HeaMcArgs& a, const HeaSearchPlan& p, hipStream_t st);
 
 // Launchers implemented in hea_mc.hip.
 size_t hea_mc_lds_bytes(int kmax, int task, int tp, int n_sites, bool sp_lds);

@@ -70,21 +70,23 @@ HEA_SCREEN_HD double replay(double v, double d1, int n1, int n2) {
 }
 
 // Exact replay of entry (a,b) for proposal (a1, a2) over one shell
-// (accelerate.cpp:517-549 restricted to the updates that hit (a,b)).
+// (accelerate.cpp:517-549 restricted to the updates that hit (a,b)).  The
+// species of a1 and a2 before the swap are a and b whatever sp holds there,
+// so the replay may run while another wave writes the swap.
+template <class Sp>
 HEA_SCREEN_HD double replay_ab(double v, double delta, const int32_t* __restrict__ r1,
-                                            const int32_t* __restrict__ r2, int z,
-                                            const uint8_t* __restrict__ sp, int a1, int a2, int a,
-                                            int b) {
+                               const int32_t* __restrict__ r2, int z, const Sp sp, int a1, int a2,
+                               int a, int b) {
   for (int k = 0; k < z; ++k) {
     const int nb = r1[k];
-    const int n = sp[nb];
+    const int n = (nb == a2) ? b : (nb == a1) ? a : (int)sp[nb];
     const int na = (nb == a2) ? a : (nb == a1) ? b : n;
     if (n == b) v = v - delta;   // gamma[a][n]  -= d
     if (na == a) v = v + delta;  // gamma[na][b] += d
   }
   for (int k = 0; k < z; ++k) {
     const int nb = r2[k];
-    const int m = sp[nb];
+    const int m = (nb == a1) ? a : (nb == a2) ? b : (int)sp[nb];
     const int ma = (nb == a1) ? b : (nb == a2) ? a : m;
     if (m == a) v = v - delta;   // gamma[m][b]  -= d
     if (ma == b) v = v + delta;  // gamma[a][ma] += d
@@ -121,6 +123,28 @@ struct EntryBounds {
   float hz;      // guided mode: Z_s |H_ij|
 };
 
+template <class Args>
+HEA_SCREEN_HD EntryBounds entry_bounds(const Args& A, int s, double q, double dij, double dji,
+                                       double c) {
+  // error bounds (each computed with a few roundings; the 1.0001 factors
+  // cover them)
+  const double z = (double)A.Z[s], delta = A.delta[s];
+  const double D1 = fabs(dij) + fabs(dji);
+  // 1/dd from the screen coefficient |c| = fl(delta/dd) and 1/delta = Z N
+  // (each within a few u; the 1.0001 factors cover them)
+  const double idd = fabs(c) * (z * (double)A.N);
+  const double Ae = (6.0 * z * delta + (6.0 * z + 4.0) * 0x1p-52) * idd * 1.0001;
+  const double e2 = (12.0 * z * kHeaU * delta + (6.0 * z + 4.0) * 0x1p-52) * idd * 1.0001;
+  const double m = 2.0 * fabs(q) + 2.0 + D1 + 3.0 * Ae;
+  const double e1 = 2.0 * kHeaU * m * 1.0001;
+  const double t1 = D1 + Ae + e1;
+  const double P = 2.0 * e2 * (D1 + Ae) + 2.0 * (Ae + e2) * (kHeaU * D1 + e2) +
+                   2.0 * e1 * (D1 + 2.0 * Ae + e1) + 2.0 * kHeaU * t1 * t1 +
+                   2.0 * kHeaU * (Ae + e2) * (D1 + Ae + e2);
+  const double ub = D1 + Ae + e1 + e2;
+  return EntryBounds{P * 1.0001, ub * 1.0001, 0.0f};
+}
+
 template <int KMAX, bool GUIDED, class Args, class Tab>
 HEA_SCREEN_HD EntryBounds refresh_entry_core(const Args& A, const Tab& T, int s, int i, int j) {
   const int e = T.idx(s, i, j);
@@ -133,23 +157,7 @@ HEA_SCREEN_HD EntryBounds refresh_entry_core(const Args& A, const Tab& T, int s,
   T.E0[e] = dij * dij;
   T.R[e] = safe_step(g, A.delta[s], A.Z[s]);
   T.SC[e].x = dij + dji;
-  // error bounds (each computed with a few roundings; the 1.0001 factors
-  // cover them)
-  const double z = (double)A.Z[s], delta = A.delta[s];
-  const double D1 = fabs(dij) + fabs(dji);
-  // 1/dd from the screen coefficient |c| = fl(delta/dd) and 1/delta = Z N
-  // (each within a few u; the 1.0001 factors cover them)
-  const double idd = fabs(T.SC[e].y) * (z * (double)A.N);
-  const double Ae = (6.0 * z * delta + (6.0 * z + 4.0) * 0x1p-52) * idd * 1.0001;
-  const double e2 = (12.0 * z * kHeaU * delta + (6.0 * z + 4.0) * 0x1p-52) * idd * 1.0001;
-  const double m = 2.0 * fabs(q) + 2.0 + D1 + 3.0 * Ae;
-  const double e1 = 2.0 * kHeaU * m * 1.0001;
-  const double t1 = D1 + Ae + e1;
-  const double P = 2.0 * e2 * (D1 + Ae) + 2.0 * (Ae + e2) * (kHeaU * D1 + e2) +
-                   2.0 * e1 * (D1 + 2.0 * Ae + e1) + 2.0 * kHeaU * t1 * t1 +
-                   2.0 * kHeaU * (Ae + e2) * (D1 + Ae + e2);
-  const double ub = D1 + Ae + e1 + e2;
-  EntryBounds r{P * 1.0001, ub * 1.0001, 0.0f};
+  EntryBounds r = entry_bounds(A, s, q, dij, dji, T.SC[e].y);
   if constexpr (GUIDED) {
     // H_ij = dF2/dn_ij + dF2/dn_ji of the fitness squared
     // (accelerate.cpp:556-569) with gamma = n delta: dF2/dn_ij =
@@ -216,12 +224,101 @@ HEA_SCREEN_HD double screen_shell(const Tab& T, int K, int s, int a, int b,
   return x;
 }
 
+// ---- the same screen on folded tables (kernels that keep T.UV) ----
+//
+// With c = -delta/dd and x = d_ij + d_ji of an entry, the shell's screen
+// value is w sum 2 net c (x + net c) over the changed entry pairs (diagonal
+// entries once).  T.UV holds u = 2 w c x and v = 2 w c^2 of every entry, so a
+// pair's value is net (u + net v), and the rows a and b of a species q other
+// than a and b, whose nets are opposite, share one term
+// net ((u_a - u_b) + net (v_a + v_b)).
+//
+// Rounding: u and v carry two roundings each, the differences and sums one,
+// the inner fma one, so each term is off by at most 4.1 units of w 4 ub^2
+// (|net c| <= A, |x| <= D1, ub >= D1 + A); the accumulation adds one rounding
+// of the running sum, at most u sum_s w_s 2K 4 ub_s^2, per term and shell
+// (S (K + 3) of them).  fold_bound charges S (K + 3) + 12 units of 4 ub^2 per
+// changed pair, 2K pairs per shell.
+
+// Half of the window half-width's share of one entry: beta of the folded
+// screen is the sum over the shells of twice the largest fold_bound (the pair
+// errors and the K^2-term sums may be largest at different entries).
+template <class Args>
+HEA_SCREEN_HD double fold_bound(const Args& A, int s, double P, double ub) {
+  const double K = (double)A.K, S = (double)A.S, u2 = kHeaU * ub * ub;
+  const double pairs = (2.0 * K) * (P + (S * (K + 3.0) + 12.0) * 4.0 * u2);
+  const double sums = (K * K) * (K * K + S + 6.0) * 1.01 * u2;
+  return fabs(A.weight[s]) * (pairs + sums);
+}
+
+// Refreshes the folded tables of entries (s,i,j) and (s,j,i), whose gamma g is
+// the same: E0, R, u (v is constant), and the bound B of both (see
+// refresh_entry_core, whose bounds these are).
+template <class Args, class Tab>
+HEA_SCREEN_HD void refresh_fold(const Args& A, const Tab& T, int s, int i, int j, double g) {
+  const int e = T.idx(s, i, j), f = T.idx(s, j, i);
+  const double dd = T.conc[i] * T.conc[j];
+  const double q = g / dd;
+  const double al = 1.0 - q;
+  const double dij = al - T.tgt[e], dji = al - T.tgt[f];
+  const double c = T.C[e];
+  const double u = (2.0 * A.weight[s] * c) * (dij + dji);
+  T.UV[T.uvx(s, i, j)].x = u;
+  T.UV[T.uvx(s, j, i)].x = u;
+  T.E0[e] = dij * dij;
+  T.E0[f] = dji * dji;
+  const double r = safe_step(g, A.delta[s], A.Z[s]);
+  T.R[e] = r;
+  T.R[f] = r;
+  const EntryBounds eb = entry_bounds(A, s, q, dij, dji, c);
+  const double b = fold_bound(A, s, eb.P, eb.ub);
+  T.B[e] = b;
+  T.B[f] = b;
+}
+
+// X of one proposal: the sum over the shells of the folded screen, for
+// swapping species a (at a1) and b (at a2) with the shells' histograms MA, MB
+// and adjacency counts c12 = c21 (symmetric relation, no self neighbours).
+template <int KMAX, class Tab>
+HEA_SCREEN_HD double screen_fold(const Tab& T, int S, int a, int b,
+                                 const typename Pack<KMAX>::T* MA,
+                                 const typename Pack<KMAX>::T* MB, const int* c12) {
+  using PK = Pack<KMAX>;
+  using PT = typename PK::T;
+  const PT field = (PT)((1u << PK::W) - 1u);
+  const PT keep = ~((field << (PK::W * a)) | (field << (PK::W * b)));
+  double X = 0.0;
+#pragma unroll
+  for (int s = 0; s < HEA_MAX_S; ++s) {
+    if (s < S) {
+      const auto* ra = T.UV + T.uvx(s, a, 0);
+      const auto* rb = T.UV + T.uvx(s, b, 0);
+      const PT ma = MA[s] & keep, mb = MB[s] & keep;
+#pragma unroll
+      for (int q = 0; q < KMAX; ++q) {  // (fields of absent species are zero)
+        const double n = (double)(PK::fld(mb, q) - PK::fld(ma, q));
+        const auto ea = ra[q], eb = rb[q];
+        X = fma(n, fma(n, ea.y + eb.y, ea.x - eb.x), X);
+      }
+      const int maA = PK::fld(MA[s], a), maB = PK::fld(MA[s], b);
+      const int mbA = PK::fld(MB[s], a), mbB = PK::fld(MB[s], b);
+      // half of nAA = 2 (mbA - c21) - 2 maA and of nBB = 2 (maB - c12) - 2 mbB
+      const double hA = (double)(mbA - c12[s] - maA), hB = (double)(maB - c12[s] - mbB);
+      const double n = (double)(maA + mbB + 2 * c12[s] - maB - mbA);
+      const auto eaa = ra[a], ebb = rb[b], eab = ra[b];
+      X = fma(hA, fma(2.0 * hA, eaa.y, eaa.x), X);
+      X = fma(hB, fma(2.0 * hB, ebb.y, ebb.x), X);
+      X = fma(n, fma(n, eab.y, eab.x), X);
+    }
+  }
+  return X;
+}
+
 // Exact new values of gamma entries (a,x) and (b,x) of shell s for swapping
 // a1 <-> a2 (species a != b), from the stored walk of the two neighbour
 // lists (file header: fast path, or replay when the entry's step is 0).
-template <int KMAX, class Args, class Tab>
-HEA_SCREEN_HD void exact_entries(const Args& A, const Tab& T,
-                                              const uint8_t* __restrict__ sp, int s, int a1,
+template <int KMAX, class Args, class Tab, class Sp>
+HEA_SCREEN_HD void exact_entries(const Args& A, const Tab& T, const Sp sp, int s, int a1,
                                               int a2, int a, int b, int x,
                                               typename Pack<KMAX>::T MA,
                                               typename Pack<KMAX>::T MB, int c11, int c12,
