@@ -662,9 +662,9 @@ void fill_problem_args(hea_problem p, HeaMcArgs& a) {
 
 // Launch of a plain search of `task` proposals a round by the stencil-lattice
 // kernel (threads = 0: the problem or round size is not for it).
-HeaSearchPlan search_plan(hea_problem p, int task) {
+HeaSearchPlan search_plan(hea_problem p, int task, bool batch = false) {
   if (p->force_hbm_species) return HeaSearchPlan();
-  return hea_search_plan(p->hc, p->lt, task, p->max_lds);
+  return hea_search_plan(p->hc, p->lt, task, p->max_lds, batch);
 }
 
 int launch_mc(hea_problem p, uint8_t* lat, double* fit, const int32_t* counts, int64_t* stats,
@@ -1445,6 +1445,11 @@ struct hea_batch_s {
   DevBuf<int64_t> stats;
   DevBuf<uint32_t> iter, queue;   // queue: [HEA_XCDS] next item of each part
   int xoff[HEA_XCDS + 1] = {};     // item parts (HeaMcBatchArgs)
+  // plain searches of a batch of several problems: the stencil problems' items
+  // (k_search_batch, longest first) and the others' (the persistent kernel)
+  DevBuf<int2> s_items, r_items;
+  int n_search = 0, n_rest = 0, s_threads = 0, r_xoff[HEA_XCDS + 1] = {};
+  size_t s_lds = 0;
   DevBuf<uint32_t> tie;            // [problems] tie flags of the population sorts
   DevBuf<unsigned long long> clk;  // [0] start, [1 + p] first fitness <= thr of problem p
   DevBuf<HeaMcArgs> margs;         // launch arguments [2 phases][problems] for population B
@@ -1491,10 +1496,11 @@ static int batch_enqueue_iteration(hea_batch b, const IterHooks* hk = nullptr) {
                      (uint32_t)HEA_PHASE_NEW);
   if ((rc = batch_recount(b))) return rc;
   hipLaunchKernelGGL(k_fitness_batch, dim3((L + 63) / 64, P), dim3(64), 0, st, b->pops.p, L);
+  const bool split = P > 1 && !b->guide.hist && b->n_search > 0;
   HeaMcBatchArgs ba;
-  ba.items = b->items.p;
-  ba.n_items = P * L;
-  for (int x = 0; x <= HEA_XCDS; ++x) ba.xoff[x] = b->xoff[x];
+  ba.items = split ? b->r_items.p : b->items.p;
+  ba.n_items = split ? b->n_rest : P * L;
+  for (int x = 0; x <= HEA_XCDS; ++x) ba.xoff[x] = split ? b->r_xoff[x] : b->xoff[x];
   ba.queue = b->queue.p;
   for (int phase = HEA_PHASE_LS1; phase <= HEA_PHASE_LS2; ++phase) {
     ba.probs = b->margs.p + (size_t)(phase - HEA_PHASE_LS1) * P;
@@ -1515,9 +1521,14 @@ static int batch_enqueue_iteration(hea_batch b, const IterHooks* hk = nullptr) {
       HEA_HIP(hea_launch_search(a, plan, st));
     } else if (P == 1)  // nothing to balance: the arguments go in the kernarg segment
       HEA_HIP(hea_launch_local_mc(b->hmargs[h], b->probs[0]->hc.K, b->sp_lds, false, b->lds, st));
-    else
-      HEA_HIP(hea_launch_local_mc_batch(ba, b->kmax, b->sp_lds, b->guide.hist != nullptr, b->grid,
-                                        b->threads, b->lds, st));
+    else {
+      if (split)
+        HEA_HIP(hea_launch_search_batch(ba.probs, b->s_items.p, b->n_search, b->s_threads,
+                                        b->s_lds, st));
+      if (ba.n_items > 0)
+        HEA_HIP(hea_launch_local_mc_batch(ba, b->kmax, b->sp_lds, b->guide.hist != nullptr,
+                                          std::min(b->grid, ba.n_items), b->threads, b->lds, st));
+    }
     if (hk) {
       HEA_HIP(hipEventRecord(hk->ev[2 * h + 1], st));
       HEA_HIP(hipMemcpyAsync(hk->snap + (h + 1) * sn, b->stats.p, sizeof(int64_t) * sn,
@@ -1602,14 +1613,28 @@ int hea_batch_create(const hea_problem* probs, int32_t n_probs, int32_t L, int32
     part[q] = x;
     load[x] += cost[q] * L;
   }
-  std::vector<int2> items;
-  for (int x = 0; x < HEA_XCDS; ++x) {
-    b->xoff[x] = (int)items.size();
-    for (int q : order)
-      if (part[q] == x)
-        for (int l = 0; l < L; ++l) items.push_back(make_int2(q, l));
+  std::vector<int2> items, s_items, r_items;
+  auto parts = [&](std::vector<int2>& to, int* xoff, const std::function<bool(int)>& take) {
+    for (int x = 0; x < HEA_XCDS; ++x) {
+      xoff[x] = (int)to.size();
+      for (int q : order)
+        if (part[q] == x && take(q))
+          for (int l = 0; l < L; ++l) to.push_back(make_int2(q, l));
+    }
+    xoff[HEA_XCDS] = (int)to.size();
+  };
+  parts(items, b->xoff, [](int) { return true; });
+  std::vector<HeaSearchPlan> plans(n_probs);
+  for (int q = 0; q < n_probs && n_probs > 1; ++q) plans[q] = search_plan(probs[q], task, true);
+  for (int q : order) {
+    if (!plans[q].threads) continue;
+    for (int l = 0; l < L; ++l) s_items.push_back(make_int2(q, l));
+    b->s_threads = plans[q].threads;  // the same for every problem: the round size sets it
+    b->s_lds = std::max(b->s_lds, plans[q].lds);
   }
-  b->xoff[HEA_XCDS] = (int)items.size();
+  parts(r_items, b->r_xoff, [&](int q) { return plans[q].threads == 0; });
+  b->n_search = (int)s_items.size();
+  b->n_rest = (int)r_items.size();
   hipError_t e = hipSuccess;
   if (e == hipSuccess) e = b->A.alloc(nl);
   if (e == hipSuccess) e = b->B.alloc(nl);
@@ -1627,6 +1652,8 @@ int hea_batch_create(const hea_problem* probs, int32_t n_probs, int32_t L, int32
   if (e == hipSuccess) e = b->merges.alloc((size_t)3 * n_probs);
   if (e == hipSuccess) e = b->pops.alloc((size_t)n_probs);
   if (e == hipSuccess) e = b->items.alloc(items.size());
+  if (e == hipSuccess) e = b->s_items.alloc(s_items.size());
+  if (e == hipSuccess) e = b->r_items.alloc(r_items.size());
   if (e == hipSuccess) e = b->tie.alloc((size_t)n_probs);
   if (e == hipSuccess) e = hipMemset(b->tie.p, 0, sizeof(uint32_t) * n_probs);
   if (e != hipSuccess) {
@@ -1652,6 +1679,7 @@ int hea_batch_create(const hea_problem* probs, int32_t n_probs, int32_t L, int32
       const int lanes = hea_mc_split(a, false);
       a.dw = hea_mc_draw_lanes(task, probs[q]->hc.conc, probs[q]->hc.K, lanes);
       b->threads = std::max(b->threads, lanes);
+      a.dl = plans[q].dl;
       a.thr = thr;
       a.seed = seed + (uint64_t)q;
       a.phase = (uint32_t)(HEA_PHASE_LS1 + ph);
@@ -1689,6 +1717,13 @@ int hea_batch_create(const hea_problem* probs, int32_t n_probs, int32_t L, int32
     e = hipMemcpy(b->pops.p, pd.data(), sizeof(HeaPopDesc) * pd.size(), hipMemcpyHostToDevice);
   if (e == hipSuccess)
     e = hipMemcpy(b->items.p, items.data(), sizeof(int2) * items.size(), hipMemcpyHostToDevice);
+  if (e == hipSuccess && !s_items.empty())
+    e = hipMemcpy(b->s_items.p, s_items.data(), sizeof(int2) * s_items.size(),
+                  hipMemcpyHostToDevice);
+  if (e == hipSuccess && !r_items.empty())
+    e = hipMemcpy(b->r_items.p, r_items.data(), sizeof(int2) * r_items.size(),
+                  hipMemcpyHostToDevice);
+  if (e == hipSuccess && b->n_search) e = hea_prepare_search_batch((size_t)probs[0]->max_lds);
   if (e == hipSuccess) e = hea_prepare_local_mc_batch(b->kmax, b->sp_lds, b->lds);
   if (e == hipSuccess && n_probs == 1)
     e = hea_prepare_local_mc(probs[0]->hc.K, b->sp_lds, false, b->lds);

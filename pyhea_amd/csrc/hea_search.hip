@@ -480,6 +480,9 @@ __device__ __forceinline__ void service_rounds(const HeaMcArgs& A, const SearchT
   SearchShared* sh = T.sh;
   const ShellArgs& SA = sh->args;
   const int K = EXACT ? KMAX : A.K, S = A.S, task = A.task, stride = A.stride;
+  const int depth = A.depth, n = A.N;
+  const double thr = A.thr;
+  const int32_t* nbr = A.nbr;
   // lane (s, h, x) takes entry (a, x) (h = 0) or (b, x) of an accepted swap
   const int sv_s = lane / (2 * K), sv_k = lane - sv_s * 2 * K;
   const int sv_h = sv_k >= K ? 1 : 0, sv_x = sv_k - sv_h * K;
@@ -488,7 +491,7 @@ __device__ __forceinline__ void service_rounds(const HeaMcArgs& A, const SearchT
   bool by_window = false;
   double beta = 0.0;
   __builtin_amdgcn_s_setprio(3);
-  for (int acc = 0, round = 0; acc < A.depth; ++round) {
+  for (int acc = 0, round = 0; acc < depth; ++round) {
     int found = 0;
     do {
       __syncthreads();  // B2
@@ -524,11 +527,11 @@ __device__ __forceinline__ void service_rounds(const HeaMcArgs& A, const SearchT
     }
     __syncthreads();  // B4
     __syncthreads();  // B1
-    d = decide(sh, nw, beta, A.thr, lane);
+    d = decide(sh, nw, beta, thr, lane);
     by_window = d.kind == 2;
     if (__builtin_expect(d.kind < 0, 0)) {
       __syncthreads();
-      undecided<KMAX, EXACT>(task, A.N, d.xmin, beta);
+      undecided<KMAX, EXACT>(task, n, d.xmin, beta);
       __syncthreads();
       read_exact(sh, T.prop, d);
       if (d.kind == 2) d.kind = 1;  // the exact stage wrote the rows in any case
@@ -549,8 +552,8 @@ __device__ __forceinline__ void service_rounds(const HeaMcArgs& A, const SearchT
     win.s1 = d.s1;
     win.s2 = d.s2;
     if (lane < stride) {
-      win.n1 = A.nbr[(size_t)d.s1 * stride + lane];
-      win.n2 = A.nbr[(size_t)d.s2 * stride + lane];
+      win.n1 = nbr[(size_t)d.s1 * stride + lane];
+      win.n2 = nbr[(size_t)d.s2 * stride + lane];
     }
   }
 }
@@ -572,7 +575,8 @@ __device__ __forceinline__ SearchCounts worker_rounds(const HeaMcArgs& A,
   uint8_t* sp = T.sp;
   const int lane = tid & 63;
   const uint32_t N = (uint32_t)A.N, nmagic = A.n_magic;
-  const int S = A.S, task = A.task;
+  const int S = A.S, task = A.task, depth = A.depth, edge = A.edge;
+  const double thr = A.thr;
   const float inv_edge = A.inv_edge;
   const auto div = [inv_edge](uint32_t n) { return hea_cell_div_small(n, inv_edge); };
   const int dl = A.dl;  // draw lanes, two consecutive draws each
@@ -609,7 +613,7 @@ __device__ __forceinline__ SearchCounts worker_rounds(const HeaMcArgs& A,
     look();
   }
 
-  for (int acc = 0; acc < A.depth;) {
+  for (int acc = 0; acc < depth;) {
     // ---- draw `task` valid proposals in stream order (accelerate.cpp:649-655)
     int found = 0;
     for (;;) {
@@ -649,7 +653,7 @@ __device__ __forceinline__ SearchCounts worker_rounds(const HeaMcArgs& A,
     {
       // (opaque: what follows from L is a few scalar instructions, not
       // registers kept over the search)
-      int L = A.edge;
+      int L = edge;
       asm("" : "+s"(L));
       const uint32_t spa = lds_addr(sp);
       const HeaCellSite ca = hea_cell_site<LT>(pr.x, L, div);
@@ -693,7 +697,7 @@ __device__ __forceinline__ SearchCounts worker_rounds(const HeaMcArgs& A,
     }
     __syncthreads();  // B1
 
-    Decision d = decide(sh, nw, beta, A.thr, lane);
+    Decision d = decide(sh, nw, beta, thr, lane);
     ++sc.rounds;
     if (__builtin_expect(d.kind < 0, 0)) {
       // the candidates of the window to the exact stage
@@ -712,7 +716,7 @@ __device__ __forceinline__ SearchCounts worker_rounds(const HeaMcArgs& A,
       __syncthreads();
       read_exact(sh, T.prop, d);
       if (d.kind == 1 && tid == 0 && A.first_hit &&
-          __longlong_as_double((long long)sh->res_key) <= A.thr)
+          __longlong_as_double((long long)sh->res_key) <= thr)
         atomicMin(A.first_hit, (unsigned long long)wall_clock64());
     }
     if (d.kind == 0) {
@@ -856,6 +860,33 @@ __global__ __launch_bounds__(kMaxSearchThreads, 4) void k_search(HeaMcArgs A) {
   search_lattice<KMAX, EXACT, LT>(A, blockIdx.x, smem);
 }
 
+// One population each of many problems: workgroup i searches lattice
+// items[i].y of problem items[i].x, longest first.  One launch for all of them,
+// so that the tail of a phase is made of short searches; table widths 4, 6 and
+// 8 (absent species hold zeros) keep the instantiations few.
+template <int LT>
+__device__ __forceinline__ void search_item(const HeaMcArgs& A, int l, unsigned char* smem) {
+  if (A.K <= 4)
+    search_lattice<4, false, LT>(A, l, smem);
+  else if (A.K <= 6)
+    search_lattice<6, false, LT>(A, l, smem);
+  else
+    search_lattice<8, false, LT>(A, l, smem);
+}
+
+__global__ __launch_bounds__(kMaxSearchThreads, 4) void k_search_batch(
+    const HeaMcArgs* __restrict__ probs, const int2* __restrict__ items) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int2 it = items[blockIdx.x];
+  const HeaMcArgs& A = probs[it.x];
+  if (A.lt == HEA_LT_FCC)
+    search_item<HEA_LT_FCC>(A, it.y, smem);
+  else if (A.lt == HEA_LT_FCC_REF)
+    search_item<HEA_LT_FCC_REF>(A, it.y, smem);
+  else
+    search_item<HEA_LT_BCC>(A, it.y, smem);
+}
+
 template <int LT>
 const void* search_fn(int K) {
   switch (K) {
@@ -892,10 +923,11 @@ size_t search_lds(int K, int task, int n) {
 
 }  // namespace
 
-HeaSearchPlan hea_search_plan(const HeaConst& c, int lt, int task, int64_t max_lds) {
+HeaSearchPlan hea_search_plan(const HeaConst& c, int lt, int task, int64_t max_lds, bool batch) {
   HeaSearchPlan p;
   if (lt == HEA_LT_NONE || task > kMaxSearchThreads - 64) return p;
-  const size_t lds = search_lds(c.K, task, c.N);
+  const int width = batch ? (c.K <= 4 ? 4 : c.K <= 6 ? 6 : 8) : c.K;
+  const size_t lds = search_lds(width, task, c.N);
   if ((int64_t)lds > max_lds) return p;
   p.lds = lds;
   const int workers = (task + 63) & ~63;
@@ -915,4 +947,16 @@ hipError_t hea_launch_search(const HeaMcArgs& a, const HeaSearchPlan& p, hipStre
   if (!fn) return hipErrorInvalidValue;
   void* args[] = {const_cast<HeaMcArgs*>(&a)};
   return hipLaunchKernel(fn, dim3(a.L), dim3(p.threads), args, p.lds, st);
+}
+
+hipError_t hea_prepare_search_batch(size_t lds) {
+  return hipFuncSetAttribute(reinterpret_cast<const void*>(k_search_batch),
+                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+}
+
+hipError_t hea_launch_search_batch(const HeaMcArgs* probs, const int2* items, int n_items,
+                                   int threads, size_t lds, hipStream_t st) {
+  void* args[] = {&probs, &items};
+  return hipLaunchKernel(reinterpret_cast<const void*>(k_search_batch), dim3(n_items),
+                         dim3(threads), args, lds, st);
 }
