@@ -737,8 +737,9 @@ int mc_lds(hea_problem p, int task, size_t* lds, bool* sp_lds, int tp = 0) {
     if ((int64_t)*lds > p->max_lds) return fail(HEA_EUNSUPPORTED, "parallel_task too large for LDS");
   }
   HEA_HIP(hea_prepare_local_mc(p->hc.K, *sp_lds, self, *lds));
-  if (search_plan(p, task).threads)
-    HEA_HIP(hea_prepare_search(p->lt, p->hc.K, (size_t)p->max_lds));
+  const HeaSearchPlan plan = search_plan(p, task);
+  if (plan.threads)
+    HEA_HIP(hea_prepare_search(p->lt, p->hc.K, plan.nib, (size_t)p->max_lds));
   return HEA_OK;
 }
 
@@ -1728,7 +1729,8 @@ int hea_batch_create(const hea_problem* probs, int32_t n_probs, int32_t L, int32
   if (e == hipSuccess && n_probs == 1)
     e = hea_prepare_local_mc(probs[0]->hc.K, b->sp_lds, false, b->lds);
   if (e == hipSuccess && n_probs == 1 && search_plan(probs[0], task).threads)
-    e = hea_prepare_search(probs[0]->lt, probs[0]->hc.K, (size_t)probs[0]->max_lds);
+    e = hea_prepare_search(probs[0]->lt, probs[0]->hc.K, search_plan(probs[0], task).nib,
+                           (size_t)probs[0]->max_lds);
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking);
   if (e != hipSuccess) {
     delete b;

@@ -145,12 +145,13 @@ __device__ __forceinline__ double hea_r_of_count(const HeaConst& P, int s, int64
 struct HeaSearchPlan {
   int threads = 0, dl = 0;
   size_t lds = 0;
+  bool nib = false;  // two species a byte
 };
 HeaSearchPlan hea_search_plan(const HeaConst& c, int lt, int task, int64_t max_lds, bool batch);
 hipError_t hea_prepare_search_batch(size_t lds);
 hipError_t hea_launch_search_batch(const HeaMcArgs* probs, const int2* items, int n_items,
                                    int threads, size_t lds, hipStream_t st);
-hipError_t hea_prepare_search(int lt, int K, size_t lds);
+hipError_t hea_prepare_search(int lt, int K, bool nib, size_t lds);
 hipError_t hea_launch_search(const HeaMcArgs& a, const HeaSearchPlan& p, hipStream_t st);
 
 // Launchers implemented in hea_mc.hip.

@@ -37,6 +37,7 @@ template <int LT>
 struct HeaShells {
   static constexpr bool BCC = LT == HEA_LT_BCC;
   static constexpr int LG = BCC ? 1 : 2, NB = 1 << LG;  // sites per cell
+  static constexpr int BIT0 = BCC ? 2 : 1;  // the axis whose parity is bit 0 of the ids
   // squared length of each shell's vectors (half units) and their number
   static constexpr int D2[3] = {BCC ? 3 : 2, 4, LT == HEA_LT_FCC ? 6 : 8};
   static constexpr int Z[3] = {BCC ? 8 : 12, 6, LT == HEA_LT_FCC ? 24 : 12};
@@ -91,12 +92,14 @@ HEA_ST_HD HeaCellSite hea_cell_site(int site, int L, const Div& div) {
   return s;
 }
 
-// f_d(V + d) for d = -2..2 of one axis at cell c and parity p.
-template <int LT, int AXIS>
+// f_d(V + d) for d = -2..2 of one axis at cell c and parity p; HALVED: of
+// id >> 1 (every term but bit 0 is even).
+template <int LT, int AXIS, bool HALVED = false>
 HEA_ST_HD void hea_axis_terms(int c, int p, int L, int* f) {
   using ST = HeaShells<LT>;
-  constexpr int B = ST::BCC ? (AXIS == 2) : AXIS;
-  const int A = AXIS == 0 ? ST::NB * L * L : AXIS == 1 ? ST::NB * L : ST::NB;
+  constexpr int B = (ST::BCC ? (AXIS == 2) : AXIS) >> (HALVED ? 1 : 0);
+  constexpr int NB = ST::NB >> (HALVED ? 1 : 0);
+  const int A = AXIS == 0 ? NB * L * L : AXIS == 1 ? NB * L : NB;
   const int at = hea_mul24(A, c), span = A * (L - 1);
   const int up = c == L - 1 ? at - span : at + A;
   const int dn = c == 0 ? at + span : at - A;

@@ -69,3 +69,19 @@ def test_equimolar_replays(gpu, counts):
     spec = make_problem("FCC", 4, None, counts=counts, target_seed=2)
     spec.target[:] = 0.0
     _check(spec, 256, 8)
+
+
+@pytest.mark.parametrize("latt,edge,shells,k,task", [
+    ("FCC", 35, "true", 5, 64), ("FCC", 36, "pyhea", 3, 33), ("BCC", 44, "true", 8, 64),
+    ("BCC", 50, "true", 2, 256),
+])
+def test_two_species_a_byte_equals_the_hbm_walk(gpu, monkeypatch, latt, edge, shells, k, task):
+    spec = make_problem(latt, edge, np.arange(3, k + 3), shells=shells, target_seed=k)
+    p = Problem.from_spec(spec)
+    monkeypatch.setenv("PYHEA_AMD_SPECIES_IN_HBM", "1")  # read when a problem is created
+    q = Problem.from_spec(spec)
+    lat, fit = p.generate(3, seed=5)
+    a = p.local_mc(lat, fit, task, 3, seed=6)
+    b = q.local_mc(lat, fit, task, 3, seed=6)
+    assert np.array_equal(a[0], b[0]) and np.array_equal(_bits(a[1]), _bits(b[1]))
+    assert all(a[2][c] == b[2][c] for c in ("evals", "rounds", "accepts", "draws"))
