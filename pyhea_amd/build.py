@@ -25,7 +25,7 @@ BUILD = os.path.join(PKG, "_build")
 LIB = os.path.join(PKG, "libpyhea_hcs.so")
 ARCH = os.environ.get("PYHEA_AMD_ARCH", "gfx950")
 
-HIP_SOURCES = ["hea_mc.hip", "hea_search.hip", "hea_search_nib.hip", "hea_api.hip",
+HIP_SOURCES = ["hea_mc.hip", "hea_search.hip", "hea_search_nib.hip", "hea_guided.hip", "hea_api.hip",
                "hea_relax.hip"]
 HIPCC_FLAGS = [
     f"--offload-arch={ARCH}",

@@ -660,6 +660,20 @@ void fill_problem_args(hea_problem p, HeaMcArgs& a) {
   a.n_magic = (uint32_t)((1ull << 32) / (uint64_t)c.N);
 }
 
+// Launch of a guided search by the stencil-lattice kernel; `a` holds the
+// launch arguments, the screen lanes (hea_mc_split) set.
+HeaSearchPlan guided_plan(hea_problem p, const HeaMcArgs& a) {
+  if (p->force_hbm_species || a.dbg_pred) return HeaSearchPlan();
+  return hea_guided_plan(p->hc, p->lt, a.task, a.g_blk, a.gbase[p->hc.S], p->max_lds);
+}
+
+// Raises the guided stencil kernels' LDS limit (before launches and captures).
+hipError_t prepare_guided(hea_problem p) {
+  if (p->lt == HEA_LT_NONE || p->hc.K > 6) return hipSuccess;
+  const hipError_t e = hea_prepare_guided(p->lt, p->hc.K, false, (size_t)p->max_lds);
+  return e != hipSuccess ? e : hea_prepare_guided(p->lt, p->hc.K, true, (size_t)p->max_lds);
+}
+
 // Launch of a plain search of `task` proposals a round by the stencil-lattice
 // kernel (threads = 0: the problem or round size is not for it).
 HeaSearchPlan search_plan(hea_problem p, int task, bool batch = false) {
@@ -704,6 +718,13 @@ int launch_mc(hea_problem p, uint8_t* lat, double* fit, const int32_t* counts, i
   }
   const HeaConst& c = p->hc;
   a.dw = hea_mc_draw_lanes(task, c.conc, c.K, hea_mc_split(a, p->hc.self_nbr != 0));
+  if (gd.hist) {
+    const HeaSearchPlan plan = guided_plan(p, a);
+    if (plan.threads) {
+      HEA_HIP(hea_launch_guided(a, plan, st));
+      return HEA_OK;
+    }
+  }
   HEA_HIP(hea_launch_local_mc(a, p->hc.K, sp_lds, p->hc.self_nbr != 0, lds, st));
   return HEA_OK;
 }
@@ -740,6 +761,7 @@ int mc_lds(hea_problem p, int task, size_t* lds, bool* sp_lds, int tp = 0) {
   const HeaSearchPlan plan = search_plan(p, task);
   if (plan.threads)
     HEA_HIP(hea_prepare_search(p->lt, p->hc.K, plan.nib, (size_t)p->max_lds));
+  HEA_HIP(prepare_guided(p));
   return HEA_OK;
 }
 
@@ -1514,9 +1536,12 @@ static int batch_enqueue_iteration(hea_batch b, const IterHooks* hk = nullptr) {
                                hipMemcpyDeviceToDevice, st));
       HEA_HIP(hipEventRecord(hk->ev[2 * h], st));
     }
-    const HeaSearchPlan plan =
-        P == 1 && !b->guide.hist ? search_plan(b->probs[0], b->task) : HeaSearchPlan();
-    if (plan.threads) {
+    const HeaSearchPlan plan = P > 1             ? HeaSearchPlan()
+                               : b->guide.hist ? guided_plan(b->probs[0], b->hmargs[h])
+                                               : search_plan(b->probs[0], b->task);
+    if (plan.threads && b->guide.hist) {
+      HEA_HIP(hea_launch_guided(b->hmargs[h], plan, st));
+    } else if (plan.threads) {
       HeaMcArgs a = b->hmargs[h];
       a.dl = plan.dl;
       HEA_HIP(hea_launch_search(a, plan, st));
@@ -1731,6 +1756,7 @@ int hea_batch_create(const hea_problem* probs, int32_t n_probs, int32_t L, int32
   if (e == hipSuccess && n_probs == 1 && search_plan(probs[0], task).threads)
     e = hea_prepare_search(probs[0]->lt, probs[0]->hc.K, search_plan(probs[0], task).nib,
                            (size_t)probs[0]->max_lds);
+  if (e == hipSuccess && n_probs == 1) e = prepare_guided(probs[0]);
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking);
   if (e != hipSuccess) {
     delete b;

@@ -145,7 +145,8 @@ __device__ __forceinline__ double hea_r_of_count(const HeaConst& P, int s, int64
 struct HeaSearchPlan {
   int threads = 0, dl = 0;
   size_t lds = 0;
-  bool nib = false;  // two species a byte
+  bool nib = false;      // two species a byte
+  bool rec_lds = false;  // guided search: neighbour records in LDS
 };
 HeaSearchPlan hea_search_plan(const HeaConst& c, int lt, int task, int64_t max_lds, bool batch);
 hipError_t hea_prepare_search_batch(size_t lds);
@@ -153,6 +154,12 @@ hipError_t hea_launch_search_batch(const HeaMcArgs* probs, const int2* items, in
                                    int threads, size_t lds, hipStream_t st);
 hipError_t hea_prepare_search(int lt, int K, bool nib, size_t lds);
 hipError_t hea_launch_search(const HeaMcArgs& a, const HeaSearchPlan& p, hipStream_t st);
+
+// The guided search on stencil lattices (hea_guided.hip).
+HeaSearchPlan hea_guided_plan(const HeaConst& c, int lt, int task, int blk, int lanes,
+                              int64_t max_lds);
+hipError_t hea_prepare_guided(int lt, int K, bool rec_lds, size_t lds);
+hipError_t hea_launch_guided(const HeaMcArgs& a, const HeaSearchPlan& p, hipStream_t st);
 
 // Launchers implemented in hea_mc.hip.
 size_t hea_mc_lds_bytes(int kmax, int task, int tp, int n_sites, bool sp_lds);

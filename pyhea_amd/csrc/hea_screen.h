@@ -253,9 +253,9 @@ HEA_SCREEN_HD double fold_bound(const Args& A, int s, double P, double ub) {
 
 // Refreshes the folded tables of entries (s,i,j) and (s,j,i), whose gamma g is
 // the same: E0, R, u (v is constant), and the bound B of both (see
-// refresh_entry_core, whose bounds these are).
+// refresh_entry_core, whose bounds these are).  Returns d_ij + d_ji.
 template <class Args, class Tab>
-HEA_SCREEN_HD void refresh_fold(const Args& A, const Tab& T, int s, int i, int j, double g) {
+HEA_SCREEN_HD double refresh_fold(const Args& A, const Tab& T, int s, int i, int j, double g) {
   const int e = T.idx(s, i, j), f = T.idx(s, j, i);
   const double dd = T.conc[i] * T.conc[j];
   const double q = g / dd;
@@ -274,6 +274,7 @@ HEA_SCREEN_HD void refresh_fold(const Args& A, const Tab& T, int s, int i, int j
   const double b = fold_bound(A, s, eb.P, eb.ub);
   T.B[e] = b;
   T.B[f] = b;
+  return dij + dji;
 }
 
 // X of one proposal: the sum over the shells of the folded screen, for

@@ -343,8 +343,8 @@ __device__ __forceinline__ uint32_t stream_mod(uint32_t w, uint32_t n, uint32_t 
 
 // Sum over the shells of twice the largest entry bound (fold_bound), by all
 // lanes of one wave.
-template <int KMAX, bool NIB>
-__device__ __forceinline__ double window(const SearchTab<KMAX, NIB>& T, int S, int K, int lane) {
+template <class Tab>
+__device__ __forceinline__ double window(const Tab& T, int S, int K, int lane) {
   if (lane < HEA_MAX_S) T.sh->vb[lane] = 0ull;
   wave_sync();
   for (int e = lane; e < S * K * K; e += 64) {
@@ -373,8 +373,8 @@ struct Winner {
 // with s >= S idle).  Entries whose step is 0 are replayed addition by
 // addition; for the interleaved entry (a, b) the rows' order of additions
 // becomes one bit mask per sign and list (a row has at most 64 columns).
-template <int KMAX, bool NIB>
-__device__ __forceinline__ double winner_entry(const ShellArgs& A, const SearchTab<KMAX, NIB>& T, int s,
+template <int KMAX, class Tab>
+__device__ __forceinline__ double winner_entry(const ShellArgs& A, const Tab& T, int s,
                                                int x, int h, int S, int stride, int a, int b,
                                                const Winner<typename Pack<KMAX>::T>& w, int lane) {
   using PK = Pack<KMAX>;
@@ -554,7 +554,7 @@ __device__ __forceinline__ void service_rounds(const HeaMcArgs& A, const SearchT
       const int r = sv_h ? d.b : d.a;
       double g = 0.0;
       if (d.kind == 2) {
-        g = winner_entry<KMAX, NIB>(SA, T, sv_s, sv_x, sv_h, S, stride, d.a, d.b, win, lane);
+        g = winner_entry<KMAX>(SA, T, sv_s, sv_x, sv_h, S, stride, d.a, d.b, win, lane);
         wave_sync();  // every lane has read its entries
         if (sv_s < S) {
           T.G[T.idx(sv_s, r, sv_x)] = g;
@@ -567,7 +567,7 @@ __device__ __forceinline__ void service_rounds(const HeaMcArgs& A, const SearchT
       wave_sync();
     }
     if (d.kind != 0 || round == 0) {
-      beta = window<KMAX, NIB>(T, S, K, lane);
+      beta = window(T, S, K, lane);
       if (lane == 0) sh->beta = beta;
     }
     __syncthreads();  // B4
