@@ -38,7 +38,7 @@
 namespace {
 
 constexpr int kPre = 12;           // candidates a lane draws ahead
-constexpr int kGroup = 2;          // candidates scored together
+constexpr int kGroup = 3;          // candidates scored together
 constexpr int kCmapWords = 1024;   // conflict map: 32768 hashed bits
 __device__ __forceinline__ uint32_t cmap_bit(int i) { return ((uint32_t)i * 0x9e3779b1u) >> 17; }
 
@@ -167,12 +167,13 @@ struct GuidedTab {
   __device__ __forceinline__ int uvx(int s, int i, int j) const { return (s * KMAX + i) * SL::KP + j; }
 };
 
-// refresh_fold and the guided tables of entries (s,i,j) and (s,j,i); returns
-// Z_s |H_ij| (refresh_entry_core's formula).
+// refresh_fold_tables and the guided tables of entries (s,i,j) and (s,j,i);
+// returns Z_s |H_ij| (refresh_entry_core's formula).
 template <int KMAX, class Tab>
 __device__ __forceinline__ float refresh_guided(const ShellArgs& A, const Tab& T, int s, int i,
                                                 int j, double g) {
-  const double D = refresh_fold(A, T, s, i, j, g);
+  const FoldEntry v = refresh_fold_tables(A, T, s, i, j, g);
+  const double D = v.dij + v.dji;
   const int e = T.idx(s, i, j), f = T.idx(s, j, i);
   T.SC[e].x = D;
   T.SC[f].x = D;
@@ -183,6 +184,19 @@ __device__ __forceinline__ float refresh_guided(const ShellArgs& A, const Tab& T
   T.HZ[e] = hz;
   T.HZ[f] = hz;
   return hz;
+}
+
+// The window of a round from its entries' bounds (fold_bound_ahead).
+__device__ __forceinline__ double round_window(const SearchShared* sh) {
+  double b = 0.0;
+#pragma unroll
+  for (int s = 0; s < HEA_MAX_S; ++s) b += __longlong_as_double((long long)sh->vb[s]);
+  return 2.0 * 1.01 * b;
+}
+
+// Largest of non-negative floats over the wave.
+__device__ __forceinline__ float fmax_all(float v) {
+  return __uint_as_float(~umin_all<true>(~__float_as_uint(v)));
 }
 
 template <int KMAX, bool RL>
@@ -225,72 +239,65 @@ __device__ __forceinline__ void guided_service(const HeaMcArgs& A, const GuidedT
   const float inv_edge = A.inv_edge;
   const auto div = [inv_edge](uint32_t x) { return hea_cell_div_small(x, inv_edge); };
   // lane (s, h, x) takes entry (a, x) (h = 0) or (b, x) of an accepted swap
-  const int sv_s = lane / (2 * K), sv_k = lane - sv_s * 2 * K;
+  // (lanes beyond them repeat an entry: they write the same values)
+  const int sv = lane % (2 * K * S);
+  const int sv_s = sv / (2 * K), sv_k = sv - sv_s * 2 * K;
   const int sv_h = sv_k >= K ? 1 : 0, sv_x = sv_k - sv_h * K;
+  // the lane's neighbour vectors: items lane and lane + 64 of [0, 2 Z), a
+  // neighbour of s1, then of s2
+  int vec[2];
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int t = lane + 64 * u;
+    vec[u] = t < 2 * Zs ? T.vec[t < Zs ? t : t - Zs] : 0;
+  }
   long long rounds = 0, accepts = 0, screens = 0;
   bool hit = false;
-  double beta = window(T, S, K, lane);
-  if (lane == 0) sh->beta = beta;
+  double beta = 0.0;
   __builtin_amdgcn_s_setprio(3);
 
-  // Accept of swap (s1: a -> b, s2: b -> a): exact rows, tables, window,
-  // species, records and the round's maps.
+  // Accept of swap (s1: a -> b, s2: b -> a): exact rows, tables, species,
+  // records and the round's maps.
   auto apply = [&](const Decision& d, const Winner<PT>& win, bool first) {
     const int r = sv_h ? d.b : d.a;
-    double g = 0.0;
+    double g;
     if (d.kind == 2) {
-      g = winner_entry<KMAX>(SA, T, sv_s, sv_x, sv_h, S, stride, d.a, d.b, win, lane);
+      g = winner_entry<KMAX>(SA, T, sv_s, sv_x, sv_h, S, stride, d.a, d.b, win, lane, [&]() {
+        int2 col = make_int2(-1, -1);
+        if (lane < stride)
+          col = make_int2(nbr[(size_t)d.s1 * stride + lane], nbr[(size_t)d.s2 * stride + lane]);
+        return col;
+      });
       wave_sync();  // every lane has read its entries
-      if (sv_s < S) {
-        T.G[T.idx(sv_s, r, sv_x)] = g;
-        T.G[T.idx(sv_s, sv_x, r)] = g;
-      }
-      if (lane == 0) {
-        sh->pfm = 2;
-        sh->fest = sh->fest + d.xmin;
-      }
-    } else if (sv_s < S) {  // the exact stage wrote its rows
+      T.G[T.idx(sv_s, r, sv_x)] = g;
+      T.G[T.idx(sv_s, sv_x, r)] = g;
+    } else {  // the exact stage wrote its rows
       g = T.G[T.idx(sv_s, r, sv_x)];
     }
-    if (first && lane == 0) sh->gmax = 0u;
-    wave_sync();
-    if (sv_s < S) {
-      const float hz = refresh_guided<KMAX>(SA, T, sv_s, r, sv_x, g);
-      if (!first) atomicMax(&sh->gmax, __float_as_uint(hz));
-    }
-    wave_sync();
-    // the first accept of a round takes the scale of every entry, the others
-    // only raise it by the entries they change
-    if (first)
-      for (int e = lane; e < S * K * K; e += 64) atomicMax(&sh->gmax, __float_as_uint(T.HZ[e]));
-    if (lane == 0) {
-      T.sp.set(d.s1, d.b);
-      T.sp.set(d.s2, d.a);
-    }
-    // item t: neighbour t of s1, then of s2
+    const float hz = refresh_guided<KMAX>(SA, T, sv_s, r, sv_x, g);
+    float top = fmax_all(hz);
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       const int t = lane + 64 * u;
-      if (t < 2 * Zs) {
-        const bool one = t < Zs;
-        const HeaCellSite c = hea_cell_site<LT>(one ? d.s1 : d.s2, L, div);
-        const int v = T.vec[one ? t : t - Zs];
-        int id = 0;
+      const bool one = t < Zs, on = t < 2 * Zs;
+      const HeaCellSite c = hea_cell_site<LT>(one ? d.s1 : d.s2, L, div);
+      int id = 0;
 #pragma unroll
-        for (int x = 0; x < 3; ++x) {
-          int V = 2 * c.c[x] + c.p[x] + ((v >> (3 * x)) & 7) - 2;
-          V = V < 0 ? V + 2 * L : V >= 2 * L ? V - 2 * L : V;
-          using ST = HeaShells<LT>;
-          const int Bx = ST::BCC ? (x == 2) : x;
-          const int Ax = x == 0 ? ST::NB * L * L : x == 1 ? ST::NB * L : ST::NB;
-          id += hea_mul24(Ax, V >> 1) + Bx * (V & 1);
-        }
-        const int s = v >> 9;
-        const int os = s == 0 ? RecBits<LT>::o(0) : s == 1 ? RecBits<LT>::o(1) : RecBits<LT>::o(2);
-        // the last species has no field (its count is implied)
-        const unsigned long long fa = d.a < K - 1 ? 1ull << (d.a * RecBits<LT>::W + os) : 0ull;
-        const unsigned long long fb = d.b < K - 1 ? 1ull << (d.b * RecBits<LT>::W + os) : 0ull;
-        const unsigned long long dv = one ? fb - fa : fa - fb;  // modulo 2^64
+      for (int x = 0; x < 3; ++x) {
+        int V = 2 * c.c[x] + c.p[x] + ((vec[u] >> (3 * x)) & 7) - 2;
+        V = V < 0 ? V + 2 * L : V >= 2 * L ? V - 2 * L : V;
+        using ST = HeaShells<LT>;
+        const int Bx = ST::BCC ? (x == 2) : x;
+        const int Ax = x == 0 ? ST::NB * L * L : x == 1 ? ST::NB * L : ST::NB;
+        id += hea_mul24(Ax, V >> 1) + Bx * (V & 1);
+      }
+      const int s = vec[u] >> 9;
+      const int os = s == 0 ? RecBits<LT>::o(0) : s == 1 ? RecBits<LT>::o(1) : RecBits<LT>::o(2);
+      // the last species has no field (its count is implied)
+      const unsigned long long fa = d.a < K - 1 ? 1ull << (d.a * RecBits<LT>::W + os) : 0ull;
+      const unsigned long long fb = d.b < K - 1 ? 1ull << (d.b * RecBits<LT>::W + os) : 0ull;
+      const unsigned long long dv = one ? fb - fa : fa - fb;  // modulo 2^64
+      if (on) {
         if constexpr (RL)
           atomicAdd(rec + id, dv);
         else
@@ -304,12 +311,28 @@ __device__ __forceinline__ void guided_service(const HeaMcArgs& A, const GuidedT
       const uint32_t mb = cmap_bit(lane == 0 ? d.s1 : d.s2);
       atomicOr(&T.cmap[mb >> 5], 1u << (mb & 31u));
     }
-    beta = window(T, S, K, lane);
+    // the first accept of a round takes the scale of every entry, the others
+    // only raise it by the entries they change
+    wave_sync();
+    if (first) {
+      for (int e = lane; e < S * K * K; e += 64) top = fmaxf(top, T.HZ[e]);
+      top = fmax_all(top);
+    }
+    if (lane == 0) {
+      T.sp.set(d.s1, d.b);
+      T.sp.set(d.s2, d.a);
+      if (d.kind == 2) {
+        sh->pfm = 2;
+        sh->fest = sh->fest + d.xmin;
+      }
+      sh->gmax = first ? __float_as_uint(top) : max(sh->gmax, __float_as_uint(top));
+    }
     wave_sync();
   };
 
   for (int acc = 0; acc < depth;) {
     __syncthreads();  // BD
+    beta = round_window(sh);
     __syncthreads();  // B1
     Decision d = decide(sh, nw, beta, thr, lane);
     ++rounds;
@@ -331,21 +354,14 @@ __device__ __forceinline__ void guided_service(const HeaMcArgs& A, const GuidedT
         reinterpret_cast<uint4*>(T.cmap)[e] = make_uint4(0, 0, 0, 0);
       for (int e = lane; e < T.bwords; e += 64) T.bmap[e] = 0u;
       Winner<PT> win{};
-      auto rows = [&]() {
-        win.s1 = d.s1;
-        win.s2 = d.s2;
-        if (lane < stride) {
-          win.n1 = nbr[(size_t)d.s1 * stride + lane];
-          win.n2 = nbr[(size_t)d.s2 * stride + lane];
-        }
-      };
-      if (sv_s < S) {
+      {
         const int w = sv_s * task + d.j;
         win.ma = T.WA[w];
         win.mb = T.WB[w];
         win.c12 = walk_unpack(T.WC[w]).c12;
+        win.s1 = d.s1;
+        win.s2 = d.s2;
       }
-      rows();
       apply(d, win, true);
       if (multi > 1) {
         __syncthreads();  // BS
@@ -405,7 +421,8 @@ __device__ __forceinline__ void guided_service(const HeaMcArgs& A, const GuidedT
           d.b = __builtin_amdgcn_readlane(b, src);
           d.s1 = __builtin_amdgcn_readlane(pr.x, src);
           d.s2 = __builtin_amdgcn_readlane(pr.y, src);
-          rows();
+          win.s1 = d.s1;
+          win.s2 = d.s2;
 #pragma unroll
           for (int s = 0; s < S; ++s) {
             const uint32_t ma = (uint32_t)__builtin_amdgcn_readlane((int)MA[s], src);
@@ -420,7 +437,7 @@ __device__ __forceinline__ void guided_service(const HeaMcArgs& A, const GuidedT
           apply(d, win, false);
         }
       }
-      if (lane == 0) sh->beta = beta;
+      if (lane < HEA_MAX_S) sh->vb[lane] = 0ull;  // the workers take the new bounds
     }
     __syncthreads();  // BA
     if (hit && lane == 0 && A.first_hit)
@@ -499,12 +516,19 @@ __device__ __forceinline__ void guided_worker(const HeaMcArgs& A, const GuidedTa
             r2[c] = load_rec<RL>(rec, by + i2);
           }
         }
+      } else {  // (or the old values stay live over the whole round)
+#pragma unroll
+        for (int c = c0; c < c0 + kGroup; ++c) {
+          noise[c] = 0.0f;
+          place[c] = 0u;
+          r1[c] = r2[c] = make_uint2(0, 0);
+        }
       }
       __builtin_amdgcn_sched_barrier(0);
     }
   };
   ahead();
-  bool changed = false;  // the last round accepted swaps
+  bool changed = false, stale = true;  // the last round accepted swaps; bounds to be taken
 
   for (int acc = 0; acc < depth;) {
     // ---- differences of the gain rows of every species pair
@@ -512,6 +536,16 @@ __device__ __forceinline__ void guided_worker(const HeaMcArgs& A, const GuidedTa
       const int p = e / (S * K), q = e - p * S * K, s = q / K, x = q - s * K;
       const int a = p / K, b = p - a * K;
       T.DH[(p * S + s) * 8 + x] = T.H[T.idx(s, b, x)] - T.H[T.idx(s, a, x)];
+    }
+    // ---- the round's window: bounds that also hold after its accepts
+    if (stale) {
+      for (int e = opaque(tid); e < S * K * K; e += nthr) {
+        const int s = e / (K * K), i = (e / K) % K, j = e % K;
+        if (i <= j) {
+          const double v = fold_bound_ahead(sh->args, T, s, i, j, T.G[e], A.g_multi);
+          atomicMax(&sh->vb[s], (unsigned long long)__double_as_longlong(v));
+        }
+      }
     }
     const float gs = 2.0f * __uint_as_float(sh->gmax);
     const float inv = (float)(1.0 / (tau * (gs > 0.0f ? (double)gs : 1.0)));
@@ -603,6 +637,7 @@ __device__ __forceinline__ void guided_worker(const HeaMcArgs& A, const GuidedTa
 
     // ---- screen the proposal (screen_shell's order of operations: the
     // shortlist is cut by X)
+    __builtin_amdgcn_sched_barrier(0);
     const int jm = opaque(j_me);
     double X = 0.0;
     {
@@ -622,11 +657,12 @@ __device__ __forceinline__ void guided_worker(const HeaMcArgs& A, const GuidedTa
         }
         X = X + sh->args.weight[s] *
                     screen_shell<KMAX, true>(T, KMAX, s, a, b, ma, mb, 0, c12, c12, 0);
+        __builtin_amdgcn_sched_barrier(0);  // one shell's table rows at a time
       });
     }
     const int2 pr = cand ? make_int2((int)s1, (int)s2) : make_int2(-1, -1);
     if (has) T.prop[jm] = pr;
-    const double beta = sh->beta;
+    const double beta = round_window(sh);
     const double xv = cand ? X : __builtin_inf();
     {
       const int src = argmin_lane<true>(xv);
@@ -659,7 +695,7 @@ __device__ __forceinline__ void guided_worker(const HeaMcArgs& A, const GuidedTa
       __syncthreads();
       d.kind = __builtin_amdgcn_readfirstlane(sh->res_kind);
     }
-    changed = d.kind != 0;
+    changed = stale = d.kind != 0;
     acc = changed ? 0 : acc + 1;
     if (changed && A.g_multi > 1) {
       // the wave's smallest X < 0, for the further accepts
@@ -706,6 +742,7 @@ __global__ __launch_bounds__(kMaxSearchThreads, 3) void k_guided(HeaMcArgs A) {
   }
   if (tid < K) T.conc[tid] = P.conc[tid];
   if (tid < kWaves) sh->wm[tid] = __builtin_inf();
+  if (tid < HEA_MAX_S) sh->vb[tid] = 0ull;
   if (tid == 0) {
     const double f0 = A.fitness[l];
     sh->pf = f0;

@@ -237,7 +237,7 @@ HEA_SCREEN_HD double screen_shell(const Tab& T, int K, int s, int a, int b,
 // the inner fma one, so each term is off by at most 4.1 units of w 4 ub^2
 // (|net c| <= A, |x| <= D1, ub >= D1 + A); the accumulation adds one rounding
 // of the running sum, at most u sum_s w_s 2K 4 ub_s^2, per term and shell
-// (S (K + 3) of them).  fold_bound charges S (K + 3) + 12 units of 4 ub^2 per
+// (at most S (K + 3) of them).  fold_bound charges S (K + 3) + 12 units of 4 ub^2 per
 // changed pair, 2K pairs per shell.
 
 // Half of the window half-width's share of one entry: beta of the folded
@@ -252,17 +252,19 @@ HEA_SCREEN_HD double fold_bound(const Args& A, int s, double P, double ub) {
 }
 
 // Refreshes the folded tables of entries (s,i,j) and (s,j,i), whose gamma g is
-// the same: E0, R, u (v is constant), and the bound B of both (see
-// refresh_entry_core, whose bounds these are).  Returns d_ij + d_ji.
+// the same: E0, R, u (v is constant).  Returns q = g/dd and d_ij, d_ji.
+struct FoldEntry {
+  double q, dij, dji;
+};
 template <class Args, class Tab>
-HEA_SCREEN_HD double refresh_fold(const Args& A, const Tab& T, int s, int i, int j, double g) {
+HEA_SCREEN_HD FoldEntry refresh_fold_tables(const Args& A, const Tab& T, int s, int i, int j,
+                                            double g) {
   const int e = T.idx(s, i, j), f = T.idx(s, j, i);
   const double dd = T.conc[i] * T.conc[j];
   const double q = g / dd;
   const double al = 1.0 - q;
   const double dij = al - T.tgt[e], dji = al - T.tgt[f];
-  const double c = T.C[e];
-  const double u = (2.0 * A.weight[s] * c) * (dij + dji);
+  const double u = (2.0 * A.weight[s] * T.C[e]) * (dij + dji);
   T.UV[T.uvx(s, i, j)].x = u;
   T.UV[T.uvx(s, j, i)].x = u;
   T.E0[e] = dij * dij;
@@ -270,11 +272,38 @@ HEA_SCREEN_HD double refresh_fold(const Args& A, const Tab& T, int s, int i, int
   const double r = safe_step(g, A.delta[s], A.Z[s]);
   T.R[e] = r;
   T.R[f] = r;
-  const EntryBounds eb = entry_bounds(A, s, q, dij, dji, c);
+  return FoldEntry{q, dij, dji};
+}
+
+// refresh_fold_tables and the bound B of both entries (see refresh_entry_core,
+// whose bounds these are).
+template <class Args, class Tab>
+HEA_SCREEN_HD void refresh_fold(const Args& A, const Tab& T, int s, int i, int j, double g) {
+  const FoldEntry v = refresh_fold_tables(A, T, s, i, j, g);
+  const int e = T.idx(s, i, j), f = T.idx(s, j, i);
+  const EntryBounds eb = entry_bounds(A, s, v.q, v.dij, v.dji, T.C[e]);
   const double b = fold_bound(A, s, eb.P, eb.ub);
   T.B[e] = b;
   T.B[f] = b;
-  return dij + dji;
+}
+
+// The bound of entry (s,i,j) for its gamma g and for every gamma that at most
+// `swaps` accepted swaps can make of it: a swap moves alpha by at most A (the
+// bound of entry_bounds: 6 Z additions of delta), so |q|, |d_ij| and |d_ji|
+// by A each.
+template <class Args, class Tab>
+HEA_SCREEN_HD double fold_bound_ahead(const Args& A, const Tab& T, int s, int i, int j, double g,
+                                      int swaps) {
+  const double dd = T.conc[i] * T.conc[j];
+  const double q = g / dd;
+  const double al = 1.0 - q, c = T.C[T.idx(s, i, j)];
+  const double z = (double)A.Z[s], idd = fabs(c) * (z * (double)A.N);
+  const double Ae = (6.0 * z * A.delta[s] + (6.0 * z + 4.0) * 0x1p-52) * idd * 1.0002;
+  const double m = (double)swaps * Ae;
+  const EntryBounds eb =
+      entry_bounds(A, s, fabs(q) + m, fabs(al - T.tgt[T.idx(s, i, j)]) + m,
+                   fabs(al - T.tgt[T.idx(s, j, i)]) + m, c);
+  return fold_bound(A, s, eb.P, eb.ub);
 }
 
 // X of one proposal: the sum over the shells of the folded screen, for
@@ -288,10 +317,11 @@ HEA_SCREEN_HD double screen_fold(const Tab& T, int S, int a, int b,
   using PT = typename PK::T;
   const PT field = (PT)((1u << PK::W) - 1u);
   const PT keep = ~((field << (PK::W * a)) | (field << (PK::W * b)));
-  double X = 0.0;
+  double sum = 0.0;
 #pragma unroll
   for (int s = 0; s < HEA_MAX_S; ++s) {
     if (s < S) {
+      double X = 0.0;  // (the shells' chains are independent)
       const auto* ra = T.UV + T.uvx(s, a, 0);
       const auto* rb = T.UV + T.uvx(s, b, 0);
       const PT ma = MA[s] & keep, mb = MB[s] & keep;
@@ -310,9 +340,10 @@ HEA_SCREEN_HD double screen_fold(const Tab& T, int S, int a, int b,
       X = fma(hA, fma(2.0 * hA, eaa.y, eaa.x), X);
       X = fma(hB, fma(2.0 * hB, ebb.y, ebb.x), X);
       X = fma(n, fma(n, eab.y, eab.x), X);
+      sum = sum + X;
     }
   }
-  return X;
+  return sum;
 }
 
 // Exact new values of gamma entries (a,x) and (b,x) of shell s for swapping

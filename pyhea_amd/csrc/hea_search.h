@@ -361,22 +361,24 @@ __device__ __forceinline__ double window(const Tab& T, int S, int K, int lane) {
 }
 
 // What the service wave keeps of a round's winner: the walk record of the
-// lane's shell, the two sites and, lane c, column c of their rows.
+// lane's shell and the two sites.
 template <class PT>
 struct Winner {
   PT ma, mb;
-  int c12, s1, s2, n1, n2;
+  int c12, s1, s2;
 };
 
 // New gamma entry (a, x) (h = 0) or (b, x) (h = 1) of shell s for the
 // winner's swap, as exact_entries gives it; by all lanes of one wave (lanes
 // with s >= S idle).  Entries whose step is 0 are replayed addition by
 // addition; for the interleaved entry (a, b) the rows' order of additions
-// becomes one bit mask per sign and list (a row has at most 64 columns).
-template <int KMAX, class Tab>
+// becomes one bit mask per sign and list (a row has at most 64 columns; rows()
+// gives lane c column c of the two sites' rows).
+template <int KMAX, class Tab, class Rows>
 __device__ __forceinline__ double winner_entry(const ShellArgs& A, const Tab& T, int s,
                                                int x, int h, int S, int stride, int a, int b,
-                                               const Winner<typename Pack<KMAX>::T>& w, int lane) {
+                                               const Winner<typename Pack<KMAX>::T>& w, int lane,
+                                               const Rows& rows) {
   using PK = Pack<KMAX>;
   double g = 0.0, r = 1.0;
   int up = 0, dn = 0, net = 0;  // additions of +delta and -delta; their sum for (a, b)
@@ -425,13 +427,14 @@ __device__ __forceinline__ double winner_entry(const ShellArgs& A, const Tab& T,
     }
     if (__any(slow && ab)) {  // replay_ab's additions in row order
       const auto sp = T.sp;
-      const bool in1 = lane < stride && w.n1 >= 0, in2 = lane < stride && w.n2 >= 0;
-      const int o1 = in1 ? sp[w.n1] : -1, o2 = in2 ? sp[w.n2] : -1;
+      const int2 col = rows();
+      const bool in1 = lane < stride && col.x >= 0, in2 = lane < stride && col.y >= 0;
+      const int o1 = in1 ? sp[col.x] : -1, o2 = in2 ? sp[col.y] : -1;
       // species before the swap, whatever sp holds at the two sites
-      const int n1 = w.n1 == w.s2 ? b : o1, n2 = w.n2 == w.s1 ? a : o2;
+      const int n1 = col.x == w.s2 ? b : o1, n2 = col.y == w.s1 ? a : o2;
       const unsigned long long m1 = __ballot(in1 && n1 == b), m2 = __ballot(in2 && n2 == a);
-      const unsigned long long p1 = __ballot(in1 && (w.n1 == w.s2 || n1 == a));
-      const unsigned long long p2 = __ballot(in2 && (w.n2 == w.s1 || n2 == b));
+      const unsigned long long p1 = __ballot(in1 && (col.x == w.s2 || n1 == a));
+      const unsigned long long p2 = __ballot(in2 && (col.y == w.s1 || n2 == b));
       const int o = on ? A.off[s] : 0;
       const uint32_t zm = on ? (1u << A.Z[s]) - 1u : 0u;
       double y = g;
@@ -532,6 +535,7 @@ __device__ __forceinline__ void service_rounds(const HeaMcArgs& A, const SearchT
   const int sv_s = lane / (2 * K), sv_k = lane - sv_s * 2 * K;
   const int sv_h = sv_k >= K ? 1 : 0, sv_x = sv_k - sv_h * K;
   Winner<typename PK::T> win{};
+  int2 col = make_int2(-1, -1);
   Decision d{};
   bool by_window = false;
   double beta = 0.0;
@@ -554,7 +558,8 @@ __device__ __forceinline__ void service_rounds(const HeaMcArgs& A, const SearchT
       const int r = sv_h ? d.b : d.a;
       double g = 0.0;
       if (d.kind == 2) {
-        g = winner_entry<KMAX>(SA, T, sv_s, sv_x, sv_h, S, stride, d.a, d.b, win, lane);
+        g = winner_entry<KMAX>(SA, T, sv_s, sv_x, sv_h, S, stride, d.a, d.b, win, lane,
+                               [&]() { return col; });
         wave_sync();  // every lane has read its entries
         if (sv_s < S) {
           T.G[T.idx(sv_s, r, sv_x)] = g;
@@ -596,10 +601,8 @@ __device__ __forceinline__ void service_rounds(const HeaMcArgs& A, const SearchT
     }
     win.s1 = d.s1;
     win.s2 = d.s2;
-    if (lane < stride) {
-      win.n1 = nbr[(size_t)d.s1 * stride + lane];
-      win.n2 = nbr[(size_t)d.s2 * stride + lane];
-    }
+    if (lane < stride)
+      col = make_int2(nbr[(size_t)d.s1 * stride + lane], nbr[(size_t)d.s2 * stride + lane]);
   }
 }
 
