@@ -239,18 +239,15 @@ __device__ __forceinline__ void guided_service(const HeaMcArgs& A, const GuidedT
   const float inv_edge = A.inv_edge;
   const auto div = [inv_edge](uint32_t x) { return hea_cell_div_small(x, inv_edge); };
   // lane (s, h, x) takes entry (a, x) (h = 0) or (b, x) of an accepted swap
-  // (lanes beyond them repeat an entry: they write the same values)
-  const int sv = lane % (2 * K * S);
-  const int sv_s = sv / (2 * K), sv_k = sv - sv_s * 2 * K;
-  const int sv_h = sv_k >= K ? 1 : 0, sv_x = sv_k - sv_h * K;
-  // the lane's neighbour vectors: items lane and lane + 64 of [0, 2 Z), a
-  // neighbour of s1, then of s2
-  int vec[2];
-#pragma unroll
-  for (int u = 0; u < 2; ++u) {
-    const int t = lane + 64 * u;
-    vec[u] = t < 2 * Zs ? T.vec[t < Zs ? t : t - Zs] : 0;
-  }
+  // (lanes beyond them repeat an entry: they write the same values).  Taken
+  // anew where it is used: kept over the rounds, what follows from it spills.
+  struct Entry {
+    int s, h, x;
+  };
+  auto entry_of = [](int ln) {
+    const int sv = opaque(ln) % (2 * K * S), k = sv % (2 * K);
+    return Entry{sv / (2 * K), k >= K ? 1 : 0, k >= K ? k - K : k};
+  };
   long long rounds = 0, accepts = 0, screens = 0;
   bool hit = false;
   double beta = 0.0;
@@ -259,6 +256,8 @@ __device__ __forceinline__ void guided_service(const HeaMcArgs& A, const GuidedT
   // Accept of swap (s1: a -> b, s2: b -> a): exact rows, tables, species,
   // records and the round's maps.
   auto apply = [&](const Decision& d, const Winner<PT>& win, bool first) {
+    const Entry en = entry_of(lane);
+    const int sv_s = en.s, sv_h = en.h, sv_x = en.x;
     const int r = sv_h ? d.b : d.a;
     double g;
     if (d.kind == 2) {
@@ -276,22 +275,24 @@ __device__ __forceinline__ void guided_service(const HeaMcArgs& A, const GuidedT
     }
     const float hz = refresh_guided<KMAX>(SA, T, sv_s, r, sv_x, g);
     float top = fmax_all(hz);
+    // items lane and lane + 64 of [0, 2 Z): a neighbour of s1, then of s2
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
-      const int t = lane + 64 * u;
+      const int t = opaque(lane) + 64 * u;
       const bool one = t < Zs, on = t < 2 * Zs;
+      const int vec = T.vec[on ? (one ? t : t - Zs) : 0];
       const HeaCellSite c = hea_cell_site<LT>(one ? d.s1 : d.s2, L, div);
       int id = 0;
 #pragma unroll
       for (int x = 0; x < 3; ++x) {
-        int V = 2 * c.c[x] + c.p[x] + ((vec[u] >> (3 * x)) & 7) - 2;
+        int V = 2 * c.c[x] + c.p[x] + ((vec >> (3 * x)) & 7) - 2;
         V = V < 0 ? V + 2 * L : V >= 2 * L ? V - 2 * L : V;
         using ST = HeaShells<LT>;
         const int Bx = ST::BCC ? (x == 2) : x;
         const int Ax = x == 0 ? ST::NB * L * L : x == 1 ? ST::NB * L : ST::NB;
         id += hea_mul24(Ax, V >> 1) + Bx * (V & 1);
       }
-      const int s = vec[u] >> 9;
+      const int s = vec >> 9;
       const int os = s == 0 ? RecBits<LT>::o(0) : s == 1 ? RecBits<LT>::o(1) : RecBits<LT>::o(2);
       // the last species has no field (its count is implied)
       const unsigned long long fa = d.a < K - 1 ? 1ull << (d.a * RecBits<LT>::W + os) : 0ull;
@@ -355,7 +356,7 @@ __device__ __forceinline__ void guided_service(const HeaMcArgs& A, const GuidedT
       for (int e = lane; e < T.bwords; e += 64) T.bmap[e] = 0u;
       Winner<PT> win{};
       {
-        const int w = sv_s * task + d.j;
+        const int w = entry_of(lane).s * task + d.j;
         win.ma = T.WA[w];
         win.mb = T.WB[w];
         win.c12 = walk_unpack(T.WC[w]).c12;
@@ -365,22 +366,24 @@ __device__ __forceinline__ void guided_service(const HeaMcArgs& A, const GuidedT
       apply(d, win, true);
       if (multi > 1) {
         __syncthreads();  // BS
-        int j = T.sl[lane];
-        const int jl = max(j, 0);
-        const int2 pr = T.prop[jl];
+        int j, c12[S], a, b;
+        int2 pr;
         PT MA[S], MB[S];
-        int c12[S], a, b;
-#pragma unroll
-        for (int s = 0; s < S; ++s) {
-          MA[s] = T.WA[s * task + jl];
-          MB[s] = T.WB[s * task + jl];
-          c12[s] = walk_unpack(T.WC[s * task + jl]).c12;
-        }
-        {
+        auto load = [&]() {  // the lane's shortlisted proposal
+          j = T.sl[opaque(lane)];
+          const int jl = max(j, 0);
+          pr = T.prop[jl];
           const WalkRec w = walk_unpack(T.WC[jl]);
           a = w.a;
           b = w.b;
-        }
+#pragma unroll
+          for (int s = 0; s < S; ++s) {
+            MA[s] = T.WA[s * task + jl];
+            MB[s] = T.WB[s * task + jl];
+            c12[s] = walk_unpack(T.WC[s * task + jl]).c12;
+          }
+        };
+        load();
         for (int step = 1; step < multi; ++step) {
           if (j >= 0) {  // a touched proposal's walk is stale: dropped for good
             const uint32_t b1 = cmap_bit(pr.x), b2 = cmap_bit(pr.y);
@@ -407,9 +410,11 @@ __device__ __forceinline__ void guided_service(const HeaMcArgs& A, const GuidedT
               T.xs[j] = X;
             }
             if (lane == 0) sh->ncl = __popcll(bal);
+            T.sl[lane] = j;
             wave_sync();
             undecided_guided<KMAX, RL>(task, n, blk, d.xmin, beta);
             wave_sync();
+            load();  // (so that the call keeps none of it)
             read_exact(sh, T.prop, d);
             if (d.kind == 2) d.kind = 1;
             if (d.kind == 1 && __longlong_as_double((long long)sh->res_key) <= thr) hit = true;
@@ -423,6 +428,7 @@ __device__ __forceinline__ void guided_service(const HeaMcArgs& A, const GuidedT
           d.s2 = __builtin_amdgcn_readlane(pr.y, src);
           win.s1 = d.s1;
           win.s2 = d.s2;
+          const int sv_s = entry_of(lane).s;
 #pragma unroll
           for (int s = 0; s < S; ++s) {
             const uint32_t ma = (uint32_t)__builtin_amdgcn_readlane((int)MA[s], src);
