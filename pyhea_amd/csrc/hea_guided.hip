@@ -256,25 +256,6 @@ __device__ __forceinline__ void guided_service(const HeaMcArgs& A, const GuidedT
   // Accept of swap (s1: a -> b, s2: b -> a): exact rows, tables, species,
   // records and the round's maps.
   auto apply = [&](const Decision& d, const Winner<PT>& win, bool first) {
-    const Entry en = entry_of(lane);
-    const int sv_s = en.s, sv_h = en.h, sv_x = en.x;
-    const int r = sv_h ? d.b : d.a;
-    double g;
-    if (d.kind == 2) {
-      g = winner_entry<KMAX>(SA, T, sv_s, sv_x, sv_h, S, stride, d.a, d.b, win, lane, [&]() {
-        int2 col = make_int2(-1, -1);
-        if (lane < stride)
-          col = make_int2(nbr[(size_t)d.s1 * stride + lane], nbr[(size_t)d.s2 * stride + lane]);
-        return col;
-      });
-      wave_sync();  // every lane has read its entries
-      T.G[T.idx(sv_s, r, sv_x)] = g;
-      T.G[T.idx(sv_s, sv_x, r)] = g;
-    } else {  // the exact stage wrote its rows
-      g = T.G[T.idx(sv_s, r, sv_x)];
-    }
-    const float hz = refresh_guided<KMAX>(SA, T, sv_s, r, sv_x, g);
-    float top = fmax_all(hz);
     // items lane and lane + 64 of [0, 2 Z): a neighbour of s1, then of s2
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
@@ -312,6 +293,27 @@ __device__ __forceinline__ void guided_service(const HeaMcArgs& A, const GuidedT
       const uint32_t mb = cmap_bit(lane == 0 ? d.s1 : d.s2);
       atomicOr(&T.cmap[mb >> 5], 1u << (mb & 31u));
     }
+    const Entry en = entry_of(lane);
+    const int sv_s = en.s, sv_h = en.h, sv_x = en.x;
+    const int r = sv_h ? d.b : d.a;
+    double g;
+    if (d.kind == 2) {
+      g = winner_entry<KMAX>(SA, T, sv_s, sv_x, sv_h, S, stride, d.a, d.b, win, lane, [&]() {
+        // (few swaps need the rows: loaded early, they wait behind the
+        // workers' record loads)
+        int2 col = make_int2(-1, -1);
+        if (lane < stride)
+          col = make_int2(nbr[(size_t)d.s1 * stride + lane], nbr[(size_t)d.s2 * stride + lane]);
+        return col;
+      });
+      wave_sync();  // every lane has read its entries
+      T.G[T.idx(sv_s, r, sv_x)] = g;
+      T.G[T.idx(sv_s, sv_x, r)] = g;
+    } else {  // the exact stage wrote its rows
+      g = T.G[T.idx(sv_s, r, sv_x)];
+    }
+    const float hz = refresh_guided<KMAX>(SA, T, sv_s, r, sv_x, g);
+    float top = fmax_all(hz);
     // the first accept of a round takes the scale of every entry, the others
     // only raise it by the entries they change
     wave_sync();
@@ -705,14 +707,26 @@ __device__ __forceinline__ void guided_worker(const HeaMcArgs& A, const GuidedTa
     acc = changed ? 0 : acc + 1;
     if (changed && A.g_multi > 1) {
       // the wave's smallest X < 0, for the further accepts
-      double v = cand && X < 0.0 ? X : __builtin_inf();
+      // (argmin_lane's keys, made once)
+      const unsigned long long xb =
+          (unsigned long long)__double_as_longlong(cand && X < 0.0 ? X : __builtin_inf());
+      const uint32_t flip = (uint32_t)((int32_t)(xb >> 32) >> 31);
+      uint32_t hi = (uint32_t)(xb >> 32) ^ (flip | 0x80000000u);
+      int mine = -1;
       for (int r = 0; r < per; ++r) {
-        const int src = argmin_lane<true>(v);
-        const double m = readlane_f64(v, src);
-        const int jr = m < 0.0 ? wave * 64 + src : -1;
-        if (lane == src) v = __builtin_inf();
-        if (lane == 0 && wave * per + r < 64) T.sl[wave * per + r] = jr;
+        const uint32_t m = umin_all<true>(hi);
+        if (m >= 0x80000000u) break;  // no X < 0 left
+        unsigned long long at = __ballot(hi == m);
+        if ((at & (at - 1ull)) != 0ull) {
+          const uint32_t lo = hi == m ? (uint32_t)xb ^ flip : ~0u;
+          const uint32_t ml = umin_all<true>(lo);
+          at = __ballot(hi == m && lo == ml);
+        }
+        const int src = (int)__builtin_ctzll(at);
+        if (lane == src) hi = ~0u;
+        if (lane == r) mine = wave * 64 + src;
       }
+      if (lane < per && wave * per + lane < 64) T.sl[wave * per + lane] = mine;
       __syncthreads();  // BS
     }
     ahead();

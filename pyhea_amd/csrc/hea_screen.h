@@ -46,20 +46,26 @@ struct Pack {
   static HEA_SCREEN_MEMBER T one(int x) { return (T)1 << (W * x); }
 };
 
-// Step r of a gamma entry valid for any sequence of <= 2*Z additions of
-// +-delta, or 0 when the entry must be replayed exactly (see file header).
-HEA_SCREEN_HD double safe_step(double g, double delta, int z) {
+// Step r of a gamma entry valid for any sequence of additions of +-delta
+// whose partial sums stay within n steps of g, or 0 when the entry must be
+// replayed exactly (see the header of hea_mc.hip).
+HEA_SCREEN_HD double safe_step_within(double g, double delta, int n) {
   if (!(g > 0.0)) return 0.0;
   int ex;
   (void)frexp(g, &ex);
   const double lo = ldexp(1.0, ex - 1), hi = ldexp(1.0, ex), u = ldexp(1.0, ex - 53);
-  const double B = (2.0 * z + 3.0) * (delta + u) * (1.0 + 0x1p-20);
+  const double B = ((double)n + 3.0) * (delta + u) * (1.0 + 0x1p-20);
   if (g - B < lo || g + B >= hi) return 0.0;
   const double t = g + delta;
   const double r = t - g;      // exact: t and g share a binade
   const double e = delta - r;  // exact (Fast2Sum, g > delta)
   if (fabs(e) == 0.5 * u) return 0.0;
   return r;
+}
+
+// The step for every swap: at most 2 Z additions either way.
+HEA_SCREEN_HD double safe_step(double g, double delta, int z) {
+  return safe_step_within(g, delta, 2 * z);
 }
 
 // Exact replay of "n1 additions of d1, then n2 additions of -d1".

@@ -381,7 +381,7 @@ __device__ __forceinline__ double winner_entry(const ShellArgs& A, const Tab& T,
                                                const Rows& rows) {
   using PK = Pack<KMAX>;
   double g = 0.0, r = 1.0;
-  int up = 0, dn = 0, net = 0;  // additions of +delta and -delta; their sum for (a, b)
+  int up = 0, dn = 0, net = 0;  // additions of +delta and -delta, and their sum
   const bool on = s < S, ab = on && x == (h ? a : b);
   if (on) {
     const int maA = PK::fld(w.ma, a), maB = PK::fld(w.ma, b);
@@ -390,7 +390,8 @@ __device__ __forceinline__ double winner_entry(const ShellArgs& A, const Tab& T,
     g = T.G[e];
     r = T.R[e];
     if (ab) {
-      net = maA + mbB + 2 * w.c12 - maB - mbA;
+      up = maA + mbB + 2 * w.c12;
+      dn = maB + mbA;
     } else {
       const bool diag = x == (h ? b : a);
       const int max_ = PK::fld(w.ma, x), mbx = PK::fld(w.mb, x);
@@ -400,13 +401,21 @@ __device__ __forceinline__ double winner_entry(const ShellArgs& A, const Tab& T,
         dn = 2 * (h ? mbB : maA);
         up = 2 * ((h ? maB : mbA) - w.c12);
       }
-      net = up - dn;
     }
+    net = up - dn;
   }
   double v = fma((double)net, r, g);
-  const bool slow = on && r == 0.0;
+  bool slow = on && r == 0.0;
+  const double delta = on ? A.delta[s] : 0.0;
   if (__any(slow)) {
-    const double delta = on ? A.delta[s] : 0.0;
+    // this swap's own additions reach less far than any swap's
+    const double rs = on ? safe_step_within(g, delta, max(up, dn)) : 0.0;
+    if (slow && rs != 0.0) {
+      v = fma((double)net, rs, g);
+      slow = false;
+    }
+  }
+  if (__any(slow)) {
     const bool plain = slow && !ab;
     // (b, x) adds first, the others subtract first
     const double d1 = h ? delta : -delta;

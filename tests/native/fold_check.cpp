@@ -5,10 +5,13 @@
 //
 //   fold_check <problem.bin> <lattices> <drift> <seed> <beta_scale>
 //   fold_check --detect <problem.bin>      prints "<shell set> <edge>"
+//   fold_check --steps <trials> <seed>     safe_step_within on random sequences
 //
 // For every unlike-species pair of random drifted lattices:
-// |err(P) - err(G) - X(P)| <= 2 beta (times <beta_scale>).  Prints
-// "ok <pairs> <max ratio>" or the first failure, exit 1.  The problem file is
+// |err(P) - err(G) - X(P)| <= 2 beta (times <beta_scale>), with beta from the
+// tables' own bounds, and again after <= 8 further swaps with beta taken before
+// them (fold_bound_ahead).  Prints "ok <pairs> <max ratio>" or the first
+// failure, exit 1.  The problem file is
 // screen_check.cpp's.
 #include <stdio.h>
 #include <stdlib.h>
@@ -46,7 +49,47 @@ bool read_all(FILE* f, void* p, size_t n) { return fread(p, 1, n, f) == n; }
 
 }  // namespace
 
+// Sequences of +-delta with partial sums within n steps of g end at
+// fma(net, r, g) whenever safe_step_within returns r != 0: random entries and
+// entries n + 3 to n + 40 steps from a binade edge, where the bound decides.
+int steps_mode(long trials, uint64_t seed) {
+  std::mt19937_64 rng(seed);
+  std::uniform_real_distribution<double> U(0.0, 1.0);
+  long fast = 0, cases = 0;
+  for (long t = 0; t < trials; ++t) {
+    const int n = 1 + (int)(rng() % 30), sites = 100 + (int)(rng() % 500000);
+    const double delta = 1.0 / (24.0 * sites);
+    const double edge = ldexp(1.0, -1 - (int)(rng() % 6));
+    const double g = (t & 1) ? edge * (1.0 + U(rng))
+                             : edge + ((rng() & 1) ? 1.0 : -1.0) * delta * (n + 40.0 * U(rng));
+    if (!(g > delta)) continue;
+    ++cases;
+    const double r = safe_step_within(g, delta, n);
+    if (r == 0.0) continue;
+    for (int q = 0; q < 4; ++q) {
+      double v = g;
+      int net = 0;
+      for (int i = 0; i < 4 * n; ++i) {
+        int st = (q == 0) ? -1 : (q == 1) ? 1 : ((rng() & 1) ? 1 : -1);
+        if (net + st > n || net + st < -n) st = -st;
+        v = st > 0 ? v + delta : v - delta;
+        net += st;
+        ++fast;
+        if (__builtin_bit_cast(uint64_t, v) !=
+            __builtin_bit_cast(uint64_t, fma((double)net, r, g))) {
+          printf("step: g %.17g delta %.17g n %d net %d\n", g, delta, n, net);
+          return 1;
+        }
+      }
+    }
+  }
+  printf("ok %ld %ld\n", cases, fast);
+  return 0;
+}
+
 int main(int argc, char** argv) {
+  if (argc == 4 && std::string(argv[1]) == "--steps")
+    return steps_mode(atol(argv[2]), strtoull(argv[3], nullptr, 10));
   const bool detect = argc == 3 && std::string(argv[1]) == "--detect";
   if (!detect && argc != 6) return 2;
   FILE* f = fopen(argv[detect ? 2 : 1], "rb");
@@ -123,6 +166,27 @@ int main(int argc, char** argv) {
       beta += most;
     }
     beta *= 2.0 * 1.01 * beta_scale;
+    // the window of a round of up to 8 further swaps, then such swaps
+    for (int round = 0; round < 2; ++round) {
+    if (round == 1) {
+      beta = 0.0;
+      for (int s = 0; s < S; ++s) {
+        double most = 0.0;
+        for (int i = 0; i < K; ++i)
+          for (int j = i; j < K; ++j)
+            most = std::max(most, fold_bound_ahead(A, T, s, i, j, g.at(i, j, s), 8));
+        beta += most;
+      }
+      beta *= 2.0 * 1.01 * beta_scale;
+      for (int d = 0; d < 8; ++d) {
+        int i = (int)(rng() % N), j = (int)(rng() % N);
+        while (lat[i] == lat[j]) j = (int)(rng() % N);
+        incremental(P, lat.data(), g, i, j);
+      }
+      for (int s = 0; s < S; ++s)
+        for (int i = 0; i < K; ++i)
+          for (int j = i; j < K; ++j) refresh_fold(A, T, s, i, j, g.at(i, j, s));
+    }
     const double errG = error_of_gamma(P, g);
     for (int a1 = 0; a1 < N; ++a1)
       for (int a2 = 0; a2 < N; ++a2) {
@@ -150,6 +214,7 @@ int main(int argc, char** argv) {
           return 1;
         }
       }
+    }
   }
   printf("ok %lld %.6g\n", pairs, max_ratio);
   return 0;

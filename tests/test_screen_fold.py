@@ -1,6 +1,7 @@
-"""The stencil-lattice search's own arithmetic on the CPU: the folded screen
+"""The stencil-lattice searches' own arithmetic on the CPU: the folded screen
 (pyhea_amd/csrc/hea_screen.h) against the oracle's sequential FP64 updates
-(its window bound, and that a bound shrunk 1e7-fold is caught), and the
+(its window bound, also the one taken for a whole round of accepts, and that a
+bound shrunk 1e7-fold is caught), the step of a bounded sequence, and the
 detection of stencil tables (hea_stencil.h): every shell set and edge it
 takes, rows in any order, and tables it must refuse."""
 import os
@@ -64,6 +65,13 @@ def test_folded_window_bound(harness, tmp_path, name):
 
 def test_shrunk_folded_window_is_caught(harness, tmp_path):
     assert all(_bound(harness, tmp_path, name, 1e-7)[0].returncode == 1 for name in CASES)
+
+
+def test_step_of_a_bounded_sequence(harness):
+    r = subprocess.run([harness, "--steps", "200000", "5"], capture_output=True, text=True)
+    assert r.returncode == 0, r.stdout + r.stderr
+    ok, cases, fast = r.stdout.split()
+    assert ok == "ok" and int(cases) > 190000 and int(fast) > 1000000
 
 
 def _detect(harness, path):
