@@ -17,12 +17,13 @@
 #include <utility>
 #include <functional>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/pyhea_hcs.h"
 #include "hea_internal.h"
 #include "hea_sort.h"
-#include "hea_stencil.h"
+#include "hea_walk.h"
 
 // Workspace of hea_local_mc_device_noalloc: the local search's iteration
 // word, per-lattice counters and pair counts live here instead of in
@@ -211,11 +212,132 @@ __device__ __forceinline__ void recount_lds_one(const HeaConst& P, const int32_t
   }
 }
 
+// Pair counts of a stencil lattice (hea_stencil.h): neighbours from
+// coordinates, and one 64-bit LDS addition per site and shell, of the counts of
+// species 0 .. K - 2 in one word, instead of one per species (their lanes meet
+// on the K rows of the table: 13 on one address for five species).  The
+// words' fields are FW bits wide and a wave's 64 sites add at most 64 x 24 to
+// one, so the wave's table goes to the workgroup's totals every FLUSH passes.
+// The counts with species K - 1 follow from the symmetry of the relation and
+// the total, Z_s N directed pairs.  512 lattices of 8192 sites: 29 us, 93 with
+// the list (its rows' loads and the additions to one address); 256 of 108000:
+// 291 us, 825 with the list.  Bound by the species gathers (42-50 a site).
+template <int KMAX, int LT>
+__device__ __forceinline__ void recount_stencil(const HeaConst& P,
+                                                const uint8_t* __restrict__ lattices,
+                                                int32_t* __restrict__ counts, int l, int edge,
+                                                float inv_edge, unsigned char* smem) {
+  using PK = Pack<KMAX>;
+  constexpr int F = KMAX - 1, FW = 64 / F < 32 ? 64 / F : 32;
+  constexpr int FLUSH = (int)(((1ull << FW) - 1ull) / (64 * 24));
+  const int K = P.K, S = P.S, N = P.N;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, nthr = blockDim.x;
+  unsigned long long* tab = reinterpret_cast<unsigned long long*>(smem);  // [waves][S][KMAX]
+  uint32_t* tot = reinterpret_cast<uint32_t*>(tab + (nthr >> 6) * HEA_MAX_S * KMAX);
+  uint8_t* sp = reinterpret_cast<uint8_t*>(tot + HEA_MAX_S * HEA_MAX_K * HEA_MAX_K);
+  unsigned long long* my = tab + wave * HEA_MAX_S * KMAX;
+  const uint8_t* lat = lattices + (size_t)l * N;
+  for (int i = tid; i < N; i += nthr) sp[i] = (uint8_t)(lat[i] * PK::W);
+  for (int e = tid; e < HEA_MAX_S * HEA_MAX_K * HEA_MAX_K; e += nthr) tot[e] = 0u;
+  if (lane < HEA_MAX_S * KMAX) my[lane] = 0ull;
+  __syncthreads();
+  const auto div = [inv_edge](uint32_t x) { return hea_cell_div_small(x, inv_edge); };
+  const uint32_t spa = lds_addr(sp);
+  auto flush = [&]() {  // by the lanes of the wave that owns the table
+    wave_sync();
+    if (lane < HEA_MAX_S * KMAX) {
+      const int s = lane / KMAX, a = lane - s * KMAX;
+      const unsigned long long v = my[lane];
+      my[lane] = 0ull;
+      if (s < S && a < K)
+        for (int x = 0; x < F && x < K - 1; ++x) {
+          const uint32_t f = (uint32_t)((v >> (x * FW)) & ((1ull << FW) - 1ull));
+          if (f) atomicAdd(&tot[(s * K + a) * K + x], f);
+        }
+    }
+    wave_sync();
+  };
+  int pass = 0;
+  for (int i0 = 0; i0 < N; i0 += nthr) {  // uniform
+    const int i = i0 + tid;
+    if (i < N) {
+      const HeaCellSite c = hea_cell_site<LT>(i, edge, div);
+      const SiteTerms t = site_terms<LT, false>(c, edge, spa);
+      const int a = Species<false, PK::W>::species_of(sp[i]);
+      auto shell = [&](auto sc, uint32_t& h) {
+        constexpr int s = decltype(sc)::value;
+        uint32_t v[HeaShells<LT>::Z[s]];
+        load_shell<LT, s>(t, v);
+        __builtin_amdgcn_sched_barrier(0);
+        h = 0;
+        count_shell<KMAX, LT, s, false>(t, v, h);
+        unsigned long long w = 0ull;
+#pragma unroll
+        for (int x = 0; x < F; ++x) w |= (unsigned long long)PK::fld(h, x) << (x * FW);
+        atomicAdd(&my[s * KMAX + a], w);
+      };
+      uint32_t h;
+      shell(std::integral_constant<int, 0>{}, h);
+      if (S > 1) shell(std::integral_constant<int, 1>{}, h);
+      if (S > 2) shell(std::integral_constant<int, 2>{}, h);
+    }
+    if (++pass == FLUSH) {
+      flush();
+      pass = 0;
+    }
+  }
+  flush();
+  __syncthreads();
+  if (tid < S) {  // the last species' row, column and diagonal
+    uint32_t* t = tot + tid * K * K;
+    uint32_t sum = 0;
+    for (int a = 0; a < K; ++a)
+      for (int x = 0; x < K - 1; ++x) sum += t[a * K + x];
+    for (int a = 0; a < K - 1; ++a) {
+      t[a * K + K - 1] = t[(K - 1) * K + a];
+      sum += t[a * K + K - 1];
+    }
+    t[K * K - 1] = (uint32_t)P.Z[tid] * (uint32_t)N - sum;
+  }
+  __syncthreads();
+  int32_t* dst = counts + (size_t)l * S * K * K;
+  for (int e = tid; e < S * K * K; e += nthr) dst[e] = (int32_t)tot[e];
+}
+
+template <int LT>
+__device__ __forceinline__ void recount_stencil_k(const HeaConst& P, const uint8_t* lattices,
+                                                  int32_t* counts, int l, int edge, float inv_edge,
+                                                  unsigned char* smem) {
+  if (P.K <= 4)
+    recount_stencil<4, LT>(P, lattices, counts, l, edge, inv_edge, smem);
+  else if (P.K == 5)
+    recount_stencil<5, LT>(P, lattices, counts, l, edge, inv_edge, smem);
+  else
+    recount_stencil<6, LT>(P, lattices, counts, l, edge, inv_edge, smem);
+}
+
+// Shell set of a problem's recount: its stencil's, or none where the counts
+// of species do not fit the words (K > 6).
+__host__ __device__ inline int recount_lt(int lt, int K) { return K <= 6 ? lt : HEA_LT_NONE; }
+
+__device__ __forceinline__ void recount_any(const HeaConst& P, const int32_t* nbr,
+                                            const uint8_t* lattices, int32_t* counts, int l, int lt,
+                                            int edge, unsigned char* smem) {
+  const float inv = edge > 0 ? 1.0f / (float)edge : 0.0f;
+  switch (recount_lt(lt, P.K)) {  // uniform
+    case HEA_LT_FCC: return recount_stencil_k<HEA_LT_FCC>(P, lattices, counts, l, edge, inv, smem);
+    case HEA_LT_FCC_REF:
+      return recount_stencil_k<HEA_LT_FCC_REF>(P, lattices, counts, l, edge, inv, smem);
+    case HEA_LT_BCC: return recount_stencil_k<HEA_LT_BCC>(P, lattices, counts, l, edge, inv, smem);
+    default: return recount_lds_one(P, nbr, lattices, counts, l, smem);
+  }
+}
+
 __global__ __launch_bounds__(kRecountLdsThreads) void k_recount_lds(
     const HeaConst* __restrict__ pc, const int32_t* __restrict__ nbr,
-    const uint8_t* __restrict__ lattices, int32_t* __restrict__ counts) {
+    const uint8_t* __restrict__ lattices, int32_t* __restrict__ counts, int lt, int edge) {
   extern __shared__ __align__(16) unsigned char smem[];
-  recount_lds_one(*pc, nbr, lattices, counts, blockIdx.x, smem);
+  recount_any(*pc, nbr, lattices, counts, blockIdx.x, lt, edge, smem);
 }
 
 size_t recount_lds_bytes(int n) {
@@ -223,30 +345,47 @@ size_t recount_lds_bytes(int n) {
 }
 
 // Fitness of freshly recounted lattices: gamma = R_s(n), then the
-// reference's sum (accelerate.cpp:165-178; std::pow(x, 2) there is x*x).
+// reference's sum (accelerate.cpp:165-178; std::pow(x, 2) there is x*x).  One
+// wave per lattice: every lane takes terms (their divisions and segment
+// searches overlap), then lane s adds shell s's terms in the reference's
+// order.  6 us at 512 lattices; one lane per lattice took 47-140 us for the
+// serial divisions.
+constexpr int kFitWaves = 4;  // lattices per workgroup
 __device__ __forceinline__ void fitness_one(const HeaConst& P, const int32_t* __restrict__ counts,
-                                            double* __restrict__ fit, int L, int l) {
-  if (l >= L) return;
-  const int K = P.K, S = P.S;
-  const int32_t* c = counts + (size_t)l * S * K * K;
-  double error = 0.0;
-  for (int s = 0; s < S; ++s) {
-    double es = 0.0;
-    for (int i = 0; i < K; ++i)
-      for (int j = 0; j < K; ++j) {
-        const double g = hea_r_of_count(P, s, c[(s * K + i) * K + j]);
-        const double sro = 1.0 - g / (P.conc[i] * P.conc[j]);
-        const double df = sro - P.target[s][i][j];
-        es = es + df * df;
-      }
-    error = error + P.weight[s] * es;
+                                            double* __restrict__ fit, int L) {
+  __shared__ double term[kFitWaves][HEA_MAX_S * HEA_MAX_K * HEA_MAX_K];
+  __shared__ double shell[kFitWaves][HEA_MAX_S];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int l = blockIdx.x * kFitWaves + wave;
+  const int K = P.K, S = P.S, E = S * K * K;
+  if (l < L) {
+    const int32_t* c = counts + (size_t)l * E;
+    for (int e = lane; e < E; e += 64) {
+      const int s = e / (K * K), i = (e / K) % K, j = e % K;
+      const double g = hea_r_of_count(P, s, c[e]);
+      const double sro = 1.0 - g / (P.conc[i] * P.conc[j]);
+      const double df = sro - P.target[s][i][j];
+      term[wave][e] = df * df;
+    }
   }
-  fit[l] = sqrt(error);
+  __syncthreads();
+  if (l < L && lane < S) {
+    double es = 0.0;
+    for (int e = 0; e < K * K; ++e) es = es + term[wave][lane * K * K + e];
+    shell[wave][lane] = es;
+  }
+  __syncthreads();
+  if (l < L && lane == 0) {
+    double error = 0.0;
+    for (int s = 0; s < S; ++s) error = error + P.weight[s] * shell[wave][s];
+    fit[l] = sqrt(error);
+  }
 }
 
-__global__ void k_fitness(const HeaConst* __restrict__ pc, const int32_t* __restrict__ counts,
-                          double* __restrict__ fit, int L) {
-  fitness_one(*pc, counts, fit, L, blockIdx.x * blockDim.x + threadIdx.x);
+__global__ __launch_bounds__(64 * kFitWaves) void k_fitness(const HeaConst* __restrict__ pc,
+                                                            const int32_t* __restrict__ counts,
+                                                            double* __restrict__ fit, int L) {
+  fitness_one(*pc, counts, fit, L);
 }
 
 // One population of every problem of a batch (problem q in the last grid
@@ -259,6 +398,7 @@ struct HeaPopDesc {
   int32_t* counts;
   double* fit;
   uint64_t seed;
+  int32_t lt, edge;
 };
 
 // k_permute over every problem; blockIdx.x of gridDim.x takes every
@@ -275,12 +415,13 @@ __global__ __launch_bounds__(kRecountLdsThreads) void k_recount_lds_batch(
     const HeaPopDesc* __restrict__ pd) {
   extern __shared__ __align__(16) unsigned char smem[];
   const HeaPopDesc d = pd[blockIdx.y];
-  recount_lds_one(*d.pc, d.nbr, d.lat, d.counts, blockIdx.x, smem);
+  recount_any(*d.pc, d.nbr, d.lat, d.counts, blockIdx.x, d.lt, d.edge, smem);
 }
 
-__global__ void k_fitness_batch(const HeaPopDesc* __restrict__ pd, int L) {
+__global__ __launch_bounds__(64 * kFitWaves) void k_fitness_batch(
+    const HeaPopDesc* __restrict__ pd, int L) {
   const HeaPopDesc d = pd[blockIdx.y];
-  fitness_one(*d.pc, d.counts, d.fit, L, blockIdx.x * blockDim.x + threadIdx.x);
+  fitness_one(*d.pc, d.counts, d.fit, L);
 }
 
 // Rank by (fitness, position) over fa[0..na) ++ fb[0..nb); writes
@@ -288,29 +429,34 @@ __global__ void k_fitness_batch(const HeaPopDesc* __restrict__ pd, int L) {
 // order (std::sort of the positions by fitness, accelerate.cpp:37-64) as
 // long as no two kept keys are equal; a kept key that equals another raises
 // *tie, and k_tie_sort then redoes the order with the reference's algorithm.
+// One wave per position: 5-8 us at 256 to 1024 keys, where one thread per
+// position, looping over all keys, took 14 to 88 us.
+constexpr int kRankWaves = 4;  // positions per workgroup
 __device__ __forceinline__ void rank_one(const double* __restrict__ fa, int na,
                                          const double* __restrict__ fb, int nb, int keep,
-                                         int32_t* __restrict__ perm, uint32_t* __restrict__ tie,
-                                         int i) {
-  const int n = na + nb;
+                                         int32_t* __restrict__ perm, uint32_t* __restrict__ tie) {
+  const int n = na + nb, lane = threadIdx.x & 63;
+  const int i = blockIdx.x * kRankWaves + (int)(threadIdx.x >> 6);
   if (i >= n) return;
   const double fi = i < na ? fa[i] : fb[i - na];
   int r = 0;
   bool eq = false;
-  for (int j = 0; j < n; ++j) {
-    const double fj = j < na ? fa[j] : fb[j - na];
-    r += (fj < fi) || (fj == fi && j < i);
-    eq |= (fj == fi) && (j != i);
+  for (int j0 = 0; j0 < n; j0 += 64) {
+    const int j = j0 + lane;
+    const double fj = j >= n ? fi : j < na ? fa[j] : fb[j - na];
+    r += __popcll(__ballot(j < n && ((fj < fi) || (fj == fi && j < i))));
+    eq |= __any(j < n && (fj == fi) && (j != i));
   }
-  if (r < keep) {
+  if (lane == 0 && r < keep) {
     perm[r] = i;
     if (eq) *tie = 1u;
   }
 }
 
-__global__ void k_rank(const double* __restrict__ fa, int na, const double* __restrict__ fb,
-                       int nb, int keep, int32_t* __restrict__ perm, uint32_t* __restrict__ tie) {
-  rank_one(fa, na, fb, nb, keep, perm, tie, blockIdx.x * blockDim.x + threadIdx.x);
+__global__ __launch_bounds__(64 * kRankWaves) void k_rank(
+    const double* __restrict__ fa, int na, const double* __restrict__ fb, int nb, int keep,
+    int32_t* __restrict__ perm, uint32_t* __restrict__ tie) {
+  rank_one(fa, na, fb, nb, keep, perm, tie);
 }
 
 // Population order on equal keys: when k_rank saw a tie, one lane sorts the
@@ -397,9 +543,10 @@ struct HeaMergeDesc {
   int32_t na, nb, keep, N;
 };
 
-__global__ void k_rank_batch(const HeaMergeDesc* __restrict__ md) {
+__global__ __launch_bounds__(64 * kRankWaves) void k_rank_batch(
+    const HeaMergeDesc* __restrict__ md) {
   const HeaMergeDesc m = md[blockIdx.y];
-  rank_one(m.fa, m.na, m.fb, m.nb, m.keep, m.perm, m.tie, blockIdx.x * blockDim.x + threadIdx.x);
+  rank_one(m.fa, m.na, m.fb, m.nb, m.keep, m.perm, m.tie);
 }
 
 __global__ __launch_bounds__(256) void k_tie_sort_batch(const HeaMergeDesc* __restrict__ md,
@@ -583,7 +730,7 @@ int launch_recount(hea_problem p, const uint8_t* lat, int32_t* counts, int L, hi
   const size_t lds = recount_lds_bytes(c.N);
   if ((int64_t)lds <= p->max_lds) {  // one workgroup per lattice, species in LDS
     hipLaunchKernelGGL(k_recount_lds, dim3(L), dim3(kRecountLdsThreads), lds, st, p->d_const.p,
-                       p->d_nbr.p, lat, counts);
+                       p->d_nbr.p, lat, counts, p->lt, p->edge);
     HEA_HIP(hipGetLastError());
     return HEA_OK;
   }
@@ -598,8 +745,8 @@ int launch_recount(hea_problem p, const uint8_t* lat, int32_t* counts, int L, hi
 }
 
 int launch_fitness(hea_problem p, const int32_t* counts, double* fit, int L, hipStream_t st) {
-  hipLaunchKernelGGL(k_fitness, dim3((L + 63) / 64), dim3(64), 0, st, p->d_const.p, counts, fit,
-                     L);
+  hipLaunchKernelGGL(k_fitness, dim3((L + kFitWaves - 1) / kFitWaves), dim3(64 * kFitWaves), 0, st,
+                     p->d_const.p, counts, fit, L);
   HEA_HIP(hipGetLastError());
   return HEA_OK;
 }
@@ -610,8 +757,8 @@ int launch_merge(const uint8_t* A, const double* fa, int na, const uint8_t* B, c
                  int nb, int keep, int32_t* perm, uint32_t* tie, uint8_t* dst, double* fdst,
                  int N, hipStream_t st) {
   const int n = na + nb;
-  hipLaunchKernelGGL(k_rank, dim3((n + 255) / 256), dim3(256), 0, st, fa, na, fb, nb, keep, perm,
-                     tie);
+  hipLaunchKernelGGL(k_rank, dim3((n + kRankWaves - 1) / kRankWaves), dim3(64 * kRankWaves), 0, st,
+                     fa, na, fb, nb, keep, perm, tie);
   const size_t tl = (size_t)n * (sizeof(double) + sizeof(int));
   const int lds = tl <= 65536 ? (int)tl : 0;
   hipLaunchKernelGGL(k_tie_sort, dim3(1), dim3(256), (size_t)lds, st, fa, na, fb, nb, keep, perm,
@@ -627,7 +774,8 @@ int launch_merge(const uint8_t* A, const double* fa, int na, const uint8_t* B, c
 // launch_merge for P problems at once: md[q] is problem q's merge; every
 // problem merges na + nb = n rows into keep, its lattices at most maxN sites.
 int launch_merge_batch(const HeaMergeDesc* md, int P, int n, int keep, int maxN, hipStream_t st) {
-  hipLaunchKernelGGL(k_rank_batch, dim3((n + 255) / 256, P), dim3(256), 0, st, md);
+  hipLaunchKernelGGL(k_rank_batch, dim3((n + kRankWaves - 1) / kRankWaves, P),
+                     dim3(64 * kRankWaves), 0, st, md);
   const size_t tl = (size_t)n * (sizeof(double) + sizeof(int));
   const int lds = tl <= 65536 ? (int)tl : 0;
   hipLaunchKernelGGL(k_tie_sort_batch, dim3(P), dim3(256), (size_t)lds, st, md, lds);
@@ -1518,7 +1666,8 @@ static int batch_enqueue_iteration(hea_batch b, const IterHooks* hk = nullptr) {
   hipLaunchKernelGGL(k_permute_batch, dim3(gx, L, P), dim3(256), 0, st, b->pops.p, b->iter.p,
                      (uint32_t)HEA_PHASE_NEW);
   if ((rc = batch_recount(b))) return rc;
-  hipLaunchKernelGGL(k_fitness_batch, dim3((L + 63) / 64, P), dim3(64), 0, st, b->pops.p, L);
+  hipLaunchKernelGGL(k_fitness_batch, dim3((L + kFitWaves - 1) / kFitWaves, P),
+                     dim3(64 * kFitWaves), 0, st, b->pops.p, L);
   const bool split = P > 1 && !b->guide.hist && b->n_search > 0;
   HeaMcBatchArgs ba;
   ba.items = split ? b->r_items.p : b->items.p;
@@ -1729,7 +1878,8 @@ int hea_batch_create(const hea_problem* probs, int32_t n_probs, int32_t L, int32
   std::vector<HeaPopDesc> pd(n_probs);
   for (int q = 0; q < n_probs; ++q)
     pd[q] = HeaPopDesc{probs[q]->d_const.p, probs[q]->d_nbr.p, b->B.p + b->lat_off[q],
-                       b->counts.p + b->cnt_off[q], b->fB.p + (size_t)q * L, seed + (uint64_t)q};
+                       b->counts.p + b->cnt_off[q], b->fB.p + (size_t)q * L, seed + (uint64_t)q,
+                       probs[q]->lt, probs[q]->edge};
   {
     const size_t lds = recount_lds_bytes(maxN);
     b->recount_lds = (int64_t)lds <= probs[0]->max_lds ? lds : 0;
