@@ -150,6 +150,13 @@ int hea_fitness(hea_problem p, int32_t solutions, const uint8_t* lattices, doubl
 /* Integer pair counts n[l][s][a][b] of each lattice (directed pairs). */
 int hea_pair_counts(hea_problem p, int32_t solutions, const uint8_t* lattices, int32_t* out);
 
+/* The same for a population stored site by site ([N][solutions], e.g. a
+ * Fortran-ordered [solutions][N] array): turned on the device. */
+int hea_fitness_columns(hea_problem p, int32_t solutions, const uint8_t* columns,
+                        double* out_fitness);
+int hea_pair_counts_columns(hea_problem p, int32_t solutions, const uint8_t* columns,
+                            int32_t* out);
+
 /* Keyed random lattices with their recount fitness: the role of
  * accelerate::cpu::generate_random_lattices (accelerate.cpp:218-252). */
 int hea_generate(hea_problem p, int32_t solutions, uint64_t seed, uint32_t iter, uint32_t phase,

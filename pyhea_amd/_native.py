@@ -29,6 +29,8 @@ EXPORTS = (
     "hea_local_mc_device_noalloc",
     "hea_fitness",
     "hea_pair_counts",
+    "hea_fitness_columns",
+    "hea_pair_counts_columns",
     "hea_generate",
     "hea_session_create",
     "hea_session_init",
@@ -111,6 +113,8 @@ def _declare(lib: C.CDLL) -> None:
         "hea_local_mc_device_noalloc": (C.c_int, [P, I32, P, P, I32, I32, U64, U32, U32, P]),
         "hea_fitness": (C.c_int, [P, I32, u8p, dp]),
         "hea_pair_counts": (C.c_int, [P, I32, u8p, i32p]),
+        "hea_fitness_columns": (C.c_int, [P, I32, u8p, dp]),
+        "hea_pair_counts_columns": (C.c_int, [P, I32, u8p, i32p]),
         "hea_generate": (C.c_int, [P, I32, U64, U32, U32, u8p, dp]),
         "hea_session_create": (C.c_int, [P, I32, I32, I32, D, U64, C.POINTER(P)]),
         "hea_session_init": (C.c_int, [P]),

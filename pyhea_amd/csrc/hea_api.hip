@@ -566,6 +566,22 @@ __global__ void k_set_u32(uint32_t* p, uint32_t v) { *p = v; }
 __global__ void k_set_u64(unsigned long long* p, unsigned long long v) { *p = v; }
 __global__ void k_clock(unsigned long long* t) { *t = wall_clock64(); }
 
+// out[l][i] = in[i][l]: a population stored site by site, in 64 x 64 tiles
+// through LDS so that both sides move whole lines.  Bound by memory: 8 MB at
+// 512 x 8192, where the host's strided copy of it took 3.6 ms.
+__global__ __launch_bounds__(256) void k_transpose_u8(const uint8_t* __restrict__ in, int N, int L,
+                                                      uint8_t* __restrict__ out) {
+  __shared__ uint8_t tile[64][65];
+  const unsigned nx = (unsigned)(N + 63) / 64;
+  const int i0 = (int)(blockIdx.x % nx) * 64, l0 = (int)(blockIdx.x / nx) * 64;
+  const int c = threadIdx.x & 63, r0 = threadIdx.x >> 6;
+  for (int r = r0; r < 64; r += 4)
+    if (i0 + r < N && l0 + c < L) tile[r][c] = in[(size_t)(i0 + r) * L + l0 + c];
+  __syncthreads();
+  for (int r = r0; r < 64; r += 4)
+    if (l0 + r < L && i0 + c < N) out[(size_t)(l0 + r) * N + i0 + c] = tile[c][r];
+}
+
 // ------------------------------------------------------------ host objects --
 
 template <typename T>
@@ -1073,29 +1089,54 @@ int hea_problem_destroy(hea_problem p) {
   return HEA_OK;
 }
 
-int hea_fitness(hea_problem p, int32_t L, const uint8_t* lattices, double* out) {
-  if (!p || L < 1 || !lattices || !out) return fail(HEA_EINVAL, "bad arguments");
+// The caller's population in p->d_lat: rows [L][N], or `cols` [N][L].
+static int upload_population(hea_problem p, int L, const uint8_t* lattices, bool cols) {
   HEA_HIP(hipSetDevice(p->device));
   int rc = ensure_scratch(p, L);
   if (rc) return rc;
-  const size_t n = (size_t)L * p->hc.N;
-  HEA_HIP(hipMemcpy(p->d_lat.p, lattices, n, hipMemcpyHostToDevice));
+  const int N = p->hc.N;
+  const size_t n = (size_t)L * N;
+  if (cols && p->d_lat2.n < n) HEA_HIP(p->d_lat2.alloc(n));
+  HEA_HIP(hipMemcpy(cols ? p->d_lat2.p : p->d_lat.p, lattices, n, hipMemcpyHostToDevice));
+  if (cols) {
+    hipLaunchKernelGGL(k_transpose_u8, dim3((unsigned)((N + 63) / 64) * (unsigned)((L + 63) / 64)),
+                       dim3(256), 0, nullptr, p->d_lat2.p, N, L, p->d_lat.p);
+    HEA_HIP(hipGetLastError());
+  }
+  return HEA_OK;
+}
+
+static int fitness_of(hea_problem p, int L, const uint8_t* lattices, bool cols, double* out) {
+  if (!p || L < 1 || !lattices || !out) return fail(HEA_EINVAL, "bad arguments");
+  int rc = upload_population(p, L, lattices, cols);
+  if (rc) return rc;
   if ((rc = launch_recount(p, p->d_lat.p, p->d_counts.p, L, nullptr))) return rc;
   if ((rc = launch_fitness(p, p->d_counts.p, p->d_fit.p, L, nullptr))) return rc;
   HEA_HIP(hipMemcpy(out, p->d_fit.p, sizeof(double) * L, hipMemcpyDeviceToHost));
   return HEA_OK;
 }
 
-int hea_pair_counts(hea_problem p, int32_t L, const uint8_t* lattices, int32_t* out) {
+static int pair_counts_of(hea_problem p, int L, const uint8_t* lattices, bool cols, int32_t* out) {
   if (!p || L < 1 || !lattices || !out) return fail(HEA_EINVAL, "bad arguments");
-  HEA_HIP(hipSetDevice(p->device));
-  int rc = ensure_scratch(p, L);
+  int rc = upload_population(p, L, lattices, cols);
   if (rc) return rc;
-  HEA_HIP(hipMemcpy(p->d_lat.p, lattices, (size_t)L * p->hc.N, hipMemcpyHostToDevice));
   if ((rc = launch_recount(p, p->d_lat.p, p->d_counts.p, L, nullptr))) return rc;
   const size_t cn = (size_t)L * p->hc.S * p->hc.K * p->hc.K;
   HEA_HIP(hipMemcpy(out, p->d_counts.p, sizeof(int32_t) * cn, hipMemcpyDeviceToHost));
   return HEA_OK;
+}
+
+int hea_fitness(hea_problem p, int32_t L, const uint8_t* lattices, double* out) {
+  return fitness_of(p, L, lattices, false, out);
+}
+int hea_fitness_columns(hea_problem p, int32_t L, const uint8_t* columns, double* out) {
+  return fitness_of(p, L, columns, true, out);
+}
+int hea_pair_counts(hea_problem p, int32_t L, const uint8_t* lattices, int32_t* out) {
+  return pair_counts_of(p, L, lattices, false, out);
+}
+int hea_pair_counts_columns(hea_problem p, int32_t L, const uint8_t* columns, int32_t* out) {
+  return pair_counts_of(p, L, columns, true, out);
 }
 
 int hea_generate(hea_problem p, int32_t L, uint64_t seed, uint32_t iter, uint32_t phase,

@@ -38,3 +38,19 @@ def test_merges_around_a_wave(gpu, solutions):
     lg, fg, _ = p.run_hcs(solutions, 2, 16, 2, seed=12)
     assert np.array_equal(lg, lo)
     assert np.array_equal(fg.view(np.uint64), fo.view(np.uint64))
+
+
+@pytest.mark.parametrize("solutions,edge", [(2, 3), (63, 4), (65, 4), (130, 5)])
+def test_populations_by_column_and_view(gpu, solutions, edge):
+    spec = make_problem("BCC", edge, [0.3, 0.3, 0.4], target_seed=3)
+    p = Problem.from_spec(spec)
+    rng = np.random.default_rng(solutions)
+    wide = rng.integers(0, 3, (2 * solutions, p.n_sites)).astype(np.uint8)
+    rows = np.ascontiguousarray(wide[::2])
+    fit, cnt = p.fitness(rows), p.pair_counts(rows)
+    for form in (np.asfortranarray(rows), wide[::2], np.asfortranarray(rows.astype(np.int64)),
+                 rows.tolist(), np.asfortranarray(wide)[::2]):
+        assert np.array_equal(p.fitness(form).view(np.uint64), fit.view(np.uint64))
+        assert np.array_equal(p.pair_counts(form), cnt)
+    with pytest.raises(ValueError):
+        p.fitness(np.asfortranarray(rows).T)
