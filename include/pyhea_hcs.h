@@ -269,7 +269,8 @@ int hea_batch_destroy(hea_batch b);
  * columns ([N][W2]; q: [S][N][W2]), zeros beyond K.  n and dn are float64
  * [S][K][K].  Asynchronous on
  * `stream`.  Calls on one problem must not overlap.  The first
- * hea_relax_forward or hea_site_gain on a problem allocates its work buffers
+ * hea_relax_forward, hea_relax_objective or hea_site_gain on a problem allocates
+ * its work buffers
  * (about 4 * N * row ints bytes) and waits for `stream` once, so it must not
  * be captured into a graph. */
 int hea_relax_forward(hea_problem p, int32_t dtype, const void* d_logits, void* d_p, void* d_q,
@@ -281,6 +282,18 @@ int32_t hea_relax_cols(int32_t n_species);
 /* Neighbour-gather adjoint: d loss / d logits from dn = d loss / d n. */
 int hea_relax_backward(hea_problem p, int32_t dtype, const void* d_p, const void* d_q,
                        const void* d_dn, void* d_grad, void* stream);
+/* hea_relax_forward and the relaxed objective in one call:
+ *   F^2 = sum_s weight_s sum_ab d^2,  d = 1 - (n_sab / zn_s) / cc_ab - target_sab,
+ * written to d_f2 (one float64), and dF^2/dn to d_dn (float64 [S][K][K]).  zn
+ * [S], cc [K][K], target [S][K][K] and weight [S] are float64 device arrays.
+ * hea_relax_backward_scaled is hea_relax_backward with dn multiplied by the
+ * float64 at d_scale (device memory; NULL: 1), so that the gradient of a loss
+ * of F^2 needs no kernel between the two. */
+int hea_relax_objective(hea_problem p, int32_t dtype, const void* d_logits, void* d_p, void* d_q,
+                        const void* d_zn, const void* d_cc, const void* d_target,
+                        const void* d_weight, void* d_f2, void* d_dn, void* stream);
+int hea_relax_backward_scaled(hea_problem p, int32_t dtype, const void* d_p, const void* d_q,
+                              const void* d_dn, const void* d_scale, void* d_grad, void* stream);
 /* Swap guidance at discrete lattices: u[l][k][b] (float32) = first-order
  * loss change of turning site k of lattice l into species b, from
  * dn[l] = d loss / d n (float64 [L][S][K][K]). */

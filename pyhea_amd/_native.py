@@ -55,6 +55,8 @@ EXPORTS = (
     "hea_batch_destroy",
     "hea_relax_forward",
     "hea_relax_backward",
+    "hea_relax_objective",
+    "hea_relax_backward_scaled",
     "hea_relax_cols",
     "hea_site_gain",
 )
@@ -142,6 +144,8 @@ def _declare(lib: C.CDLL) -> None:
         "hea_batch_destroy": (C.c_int, [P]),
         "hea_relax_forward": (C.c_int, [P, I32, P, P, P, P, P]),
         "hea_relax_backward": (C.c_int, [P, I32, P, P, P, P, P]),
+        "hea_relax_objective": (C.c_int, [P, I32] + [P] * 10),
+        "hea_relax_backward_scaled": (C.c_int, [P, I32] + [P] * 6),
         "hea_relax_cols": (I32, [I32]),
         "hea_site_gain": (C.c_int, [P, I32, P, P, P, P]),
     }

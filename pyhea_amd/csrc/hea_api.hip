@@ -637,6 +637,8 @@ struct hea_problem_s {
   // of the neighbour table
   DevBuf<double> d_relax_part;
   DevBuf<int32_t> d_relax_nbrT;
+  DevBuf<double> d_relax_n;        // pair counts of the objective's last forward
+  DevBuf<uint32_t> d_relax_ticket; // finished workgroups of the objective (zero between calls)
 };
 
 struct hea_session_s {
@@ -2217,11 +2219,12 @@ int hea_batch_destroy(hea_batch b) {
 
 // ------------------------------------------------------------- relaxation --
 hipError_t hea_relax_forward_impl(const HeaConst* dc, const HeaConst& hc, const int32_t* nbrT,
-                                  int dtype, const void* th, void* p, void* Q, double* part,
-                                  double* n, hipStream_t st);
+                                  HeaLatticeArg la, int dtype, const void* th, void* p, void* Q,
+                                  double* part, double* n, const HeaObjectiveArg* ob,
+                                  hipStream_t st);
 hipError_t hea_relax_backward_impl(const HeaConst* dc, const HeaConst& hc, int dtype,
-                                   const void* p, const void* Q, const double* dn, void* grad,
-                                   hipStream_t st);
+                                   const void* p, const void* Q, const double* dn,
+                                   const double* scale, void* grad, hipStream_t st);
 hipError_t hea_site_gain_impl(const HeaConst* dc, const HeaConst& hc, const int32_t* nbrT,
                               const uint8_t* lattices, int L, const double* dn, float* u,
                               hipStream_t st);
@@ -2235,6 +2238,9 @@ static int relax_prepare(hea_problem p, hipStream_t st) {
   if (p->d_relax_nbrT.p) return HEA_OK;
   const HeaConst& c = p->hc;
   HEA_HIP(p->d_relax_part.alloc(hea_relax_part_size(c.N, c.K, c.S)));
+  HEA_HIP(p->d_relax_n.alloc((size_t)c.S * c.K * c.K));
+  HEA_HIP(p->d_relax_ticket.alloc(1));
+  HEA_HIP(hipMemsetAsync(p->d_relax_ticket.p, 0, sizeof(uint32_t), st));
   DevBuf<int32_t> t;
   HEA_HIP(t.alloc((size_t)c.N * c.stride));
   HEA_HIP(hea_relax_transpose_nbr(p->d_nbr.p, c.N, c.stride, t.p, st));
@@ -2245,6 +2251,10 @@ static int relax_prepare(hea_problem p, hipStream_t st) {
 }
 
 extern "C" {
+
+static HeaLatticeArg lattice_arg(hea_problem p) {
+  return HeaLatticeArg{p->lt, p->edge, p->edge > 0 ? hea_cell_magic(p->edge) : 0u};
+}
 
 // Padded p and q rows are read and written as 16-byte vectors.
 static bool aligned16(const void* a) { return (reinterpret_cast<uintptr_t>(a) & 15) == 0; }
@@ -2258,21 +2268,51 @@ int hea_relax_forward(hea_problem p, int32_t dtype, const void* d_logits, void* 
   const HeaConst& c = p->hc;
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (int rc = relax_prepare(p, st)) return rc;
-  HEA_HIP(hea_relax_forward_impl(p->d_const.p, c, p->d_relax_nbrT.p, dtype, d_logits, d_p, d_q,
-                                 p->d_relax_part.p, static_cast<double*>(d_n), st));
+  HEA_HIP(hea_relax_forward_impl(p->d_const.p, c, p->d_relax_nbrT.p, lattice_arg(p), dtype,
+                                 d_logits, d_p, d_q, p->d_relax_part.p, static_cast<double*>(d_n),
+                                 nullptr, st));
   return HEA_OK;
 }
 
-int hea_relax_backward(hea_problem p, int32_t dtype, const void* d_p, const void* d_q,
-                       const void* d_dn, void* d_grad, void* stream) {
+int hea_relax_objective(hea_problem p, int32_t dtype, const void* d_logits, void* d_p, void* d_q,
+                        const void* d_zn, const void* d_cc, const void* d_target,
+                        const void* d_weight, void* d_f2, void* d_dn, void* stream) {
+  if (!p || !d_logits || !d_p || !d_q || !d_zn || !d_cc || !d_target || !d_weight || !d_f2 ||
+      !d_dn || (dtype != 0 && dtype != 1))
+    return fail(HEA_EINVAL, "bad arguments");
+  if (!aligned16(d_p) || !aligned16(d_q)) return fail(HEA_EINVAL, "p and q must be 16-byte aligned");
+  HEA_HIP(hipSetDevice(p->device));
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  if (int rc = relax_prepare(p, st)) return rc;
+  HeaObjectiveArg ob;
+  ob.zn = static_cast<const double*>(d_zn);
+  ob.cc = static_cast<const double*>(d_cc);
+  ob.target = static_cast<const double*>(d_target);
+  ob.weight = static_cast<const double*>(d_weight);
+  ob.ticket = p->d_relax_ticket.p;
+  ob.f2 = static_cast<double*>(d_f2);
+  ob.dn = static_cast<double*>(d_dn);
+  HEA_HIP(hea_relax_forward_impl(p->d_const.p, p->hc, p->d_relax_nbrT.p, lattice_arg(p), dtype,
+                                 d_logits, d_p, d_q, p->d_relax_part.p, p->d_relax_n.p, &ob, st));
+  return HEA_OK;
+}
+
+int hea_relax_backward_scaled(hea_problem p, int32_t dtype, const void* d_p, const void* d_q,
+                              const void* d_dn, const void* d_scale, void* d_grad, void* stream) {
   if (!p || !d_p || !d_q || !d_dn || !d_grad || (dtype != 0 && dtype != 1))
     return fail(HEA_EINVAL, "bad arguments");
   if (!aligned16(d_p) || !aligned16(d_q)) return fail(HEA_EINVAL, "p and q must be 16-byte aligned");
   HEA_HIP(hipSetDevice(p->device));
   HEA_HIP(hea_relax_backward_impl(p->d_const.p, p->hc, dtype, d_p, d_q,
-                                  static_cast<const double*>(d_dn), d_grad,
+                                  static_cast<const double*>(d_dn),
+                                  static_cast<const double*>(d_scale), d_grad,
                                   static_cast<hipStream_t>(stream)));
   return HEA_OK;
+}
+
+int hea_relax_backward(hea_problem p, int32_t dtype, const void* d_p, const void* d_q,
+                       const void* d_dn, void* d_grad, void* stream) {
+  return hea_relax_backward_scaled(p, dtype, d_p, d_q, d_dn, nullptr, d_grad, stream);
 }
 
 int hea_site_gain(hea_problem p, int32_t L, const void* d_lattices, const void* d_dn, void* d_u,

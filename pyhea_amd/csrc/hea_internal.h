@@ -140,6 +140,18 @@ __device__ __forceinline__ double hea_r_of_count(const HeaConst& P, int s, int64
   return fma((double)(k - P.seg_k0[s][q]), P.seg_inc[s][q], P.seg_v0[s][q]);
 }
 
+// A problem's stencil lattice (hea_stencil.h) as a kernel argument, and the
+// constants, outputs and counter of the relaxed objective (device memory).
+struct HeaLatticeArg {
+  int32_t lt, edge;
+  uint32_t magic;  // hea_cell_magic(edge)
+};
+struct HeaObjectiveArg {
+  const double *zn, *cc, *target, *weight;  // [S], [K][K], [S][K][K], [S]
+  uint32_t* ticket;                         // zero between calls
+  double *f2, *dn;                          // F^2 and dF^2/dn [S][K][K]
+};
+
 // Launch of the stencil-lattice search (hea_search.hip); threads = 0: not for
 // this problem and round size.
 struct HeaSearchPlan {

@@ -21,9 +21,10 @@
 // site's p row is 4 + W2 elements (hea_relax_cols), so K = 5 moves 5 values
 // per row, not 8.  The gather reads a neighbour's part as one vector load
 // (16 bytes for part A in float32), with the lanes of a wave all on the
-// same part, and reads the neighbour indices from a slot-major copy of the
-// table (nbrT[column][site]), one contiguous run per wave; the adjoint reads
-// Q and p rows as vectors too.
+// same part, and takes the neighbour indices from the site's coordinates on a
+// stencil lattice and else from a slot-major copy of the table
+// (nbrT[column][site]), one contiguous run per wave; the adjoint reads Q and p
+// rows as vectors too.
 // Backward (neighbour-gather adjoint): the neighbour relation is symmetric,
 // so dn[s][a][b]/dp[k][c] = [a=c] Q_s[k][b] + [b=c] Q_s[k][a] and
 //     g[k][c] = sum_s sum_b (dn[s][c][b] + dn[s][b][c]) Q_s[k][b],
@@ -36,6 +37,7 @@
 // of turning site k from its species a_k into b.
 
 #include "hea_internal.h"
+#include "hea_stencil.h"
 
 namespace {
 
@@ -105,34 +107,64 @@ __global__ __launch_bounds__(kSoftmaxThreads) void k_softmax(const T* __restrict
   }
 }
 
+// Neighbour indices of site i from the slot-major table: shell s's lists in
+// list order.
+struct TableNbrs {
+  const int32_t* nbrT;
+  int N, i;
+  const int32_t* col;
+  __device__ __forceinline__ void shell(const HeaConst& P, int s) {
+    col = nbrT + (size_t)P.off[s] * N + i;
+  }
+  __device__ __forceinline__ int operator()(int k) const { return col[(size_t)k * N]; }
+};
+
 // One gather lane: site i's own occupancies of one row part (V columns,
 // rows of V elements from `rows`) into LDS, and for every shell the sum of
 // its neighbours' rows in list order into LDS and Q (part rows of V from
 // `qrows`, shell s at qrows + s N V).
 template <typename T, int V, int KPL>
-__device__ __forceinline__ void gather_part(const HeaConst& P, const int32_t* __restrict__ nbrT,
-                                            const T* __restrict__ rows, T* __restrict__ qrows,
-                                            int i, int SB, int il, int col0, T* sp, T* sq) {
+struct GatherLane {
   using Vec = VecT<T, V>;
-  const int N = P.N, S = P.S;
-  T* myp = sp + il * KPL + col0;
-  const Vec own = *reinterpret_cast<const Vec*>(rows + (size_t)i * V);
+  const T* __restrict__ rows;
+  T* __restrict__ qrows;
+  int N, SB, i, il, col0;
+  T *sp, *sq;
+  __device__ __forceinline__ Vec row(int j) const {
+    return *reinterpret_cast<const Vec*>(rows + (size_t)j * V);
+  }
+  __device__ __forceinline__ void own() const {
+    T* myp = sp + il * KPL + col0;
+    const Vec o = row(i);
 #pragma unroll
-  for (int v = 0; v < V; ++v) myp[v] = own.x[v];
-  for (int s = 0; s < S; ++s) {
-    const int32_t* col = nbrT + (size_t)P.off[s] * N + i;
+    for (int v = 0; v < V; ++v) myp[v] = o.x[v];
+  }
+  __device__ __forceinline__ void put(int s, const double* acc) const {
+    Vec qv;
+#pragma unroll
+    for (int v = 0; v < V; ++v) qv.x[v] = (T)acc[v];
+    T* myq = sq + s * SB * KPL + il * KPL + col0;
+#pragma unroll
+    for (int v = 0; v < V; ++v) myq[v] = qv.x[v];
+    *reinterpret_cast<Vec*>(qrows + ((size_t)s * N + i) * V) = qv;
+  }
+};
+
+template <typename T, int V, int KPL>
+__device__ __forceinline__ void gather_table(const HeaConst& P, TableNbrs nb,
+                                             const GatherLane<T, V, KPL>& G) {
+  using Vec = VecT<T, V>;
+  G.own();
+  for (int s = 0; s < P.S; ++s) {
+    nb.shell(P, s);
     const int Z = P.Z[s];
     double acc[V];
 #pragma unroll
     for (int v = 0; v < V; ++v) acc[v] = 0.0;
     int k = 0;
     for (; k + 4 <= Z; k += 4) {
-      const int j0 = col[(size_t)k * N], j1 = col[(size_t)(k + 1) * N];
-      const int j2 = col[(size_t)(k + 2) * N], j3 = col[(size_t)(k + 3) * N];
-      const Vec v0 = *reinterpret_cast<const Vec*>(rows + (size_t)j0 * V);
-      const Vec v1 = *reinterpret_cast<const Vec*>(rows + (size_t)j1 * V);
-      const Vec v2 = *reinterpret_cast<const Vec*>(rows + (size_t)j2 * V);
-      const Vec v3 = *reinterpret_cast<const Vec*>(rows + (size_t)j3 * V);
+      const int j0 = nb(k), j1 = nb(k + 1), j2 = nb(k + 2), j3 = nb(k + 3);
+      const Vec v0 = G.row(j0), v1 = G.row(j1), v2 = G.row(j2), v3 = G.row(j3);
 #pragma unroll
       for (int v = 0; v < V; ++v) {
         acc[v] += (double)v0.x[v];
@@ -142,18 +174,75 @@ __device__ __forceinline__ void gather_part(const HeaConst& P, const int32_t* __
       }
     }
     for (; k < Z; ++k) {
-      const Vec vk = *reinterpret_cast<const Vec*>(rows + (size_t)col[(size_t)k * N] * V);
+      const Vec vk = G.row(nb(k));
 #pragma unroll
       for (int v = 0; v < V; ++v) acc[v] += (double)vk.x[v];
     }
-    Vec qv;
-#pragma unroll
-    for (int v = 0; v < V; ++v) qv.x[v] = (T)acc[v];
-    T* myq = sq + s * SB * KPL + il * KPL + col0;
-#pragma unroll
-    for (int v = 0; v < V; ++v) myq[v] = qv.x[v];
-    *reinterpret_cast<Vec*>(qrows + ((size_t)s * N + i) * V) = qv;
+    G.put(s, acc);
   }
+}
+
+// The same on a stencil lattice (hea_stencil.h): the neighbours' ids follow
+// from the site's coordinates, so half of the gather's load instructions, the
+// index loads, and their traffic (84 MB at 500000 sites) are gone.  Shells are
+// summed in the order of their vectors.  500000 sites, K = 6, float32: 50.7 us,
+// 55.7 with the table; 108000, K = 5: 16.7 and 19.0; 4000, K = 4, float64: 17.7
+// and 19.8.  What bounds the largest is the L1's line rate: a wave's 64 rows lie
+// in 64 lines, 47 cycles a load; the smallest has 8 workgroups.
+template <int LT, int SHELL, typename T, int V, int KPL>
+__device__ __forceinline__ void gather_shell(const int f[3][5], const GatherLane<T, V, KPL>& G) {
+  constexpr int Z = HeaShells<LT>::Z[SHELL];
+  constexpr int B = 6;  // rows in flight (6 divides every shell but BCC's 8)
+  int id[Z];
+  int n = 0;
+#pragma unroll
+  for (int dx = -2; dx <= 2; ++dx)
+#pragma unroll
+    for (int dy = -2; dy <= 2; ++dy)
+#pragma unroll
+      for (int dz = -2; dz <= 2; ++dz)
+        if (HeaShells<LT>::shell(dx, dy, dz) == SHELL)
+          id[n++] = f[0][dx + 2] + f[1][dy + 2] + f[2][dz + 2];
+  double acc[V];
+#pragma unroll
+  for (int v = 0; v < V; ++v) acc[v] = 0.0;
+#pragma unroll
+  for (int k0 = 0; k0 < Z; k0 += B) {
+    VecT<T, V> r[B];
+#pragma unroll
+    for (int k = 0; k < B; ++k)
+      if (k0 + k < Z) r[k] = G.row(id[k0 + k]);
+#pragma unroll
+    for (int k = 0; k < B; ++k)
+      if (k0 + k < Z) {
+#pragma unroll
+        for (int v = 0; v < V; ++v) acc[v] += (double)r[k].x[v];
+      }
+  }
+  G.put(SHELL, acc);
+}
+template <int LT, typename T, int V, int KPL>
+__device__ __forceinline__ void gather_stencil(const HeaConst& P, HeaLatticeArg la,
+                                               const GatherLane<T, V, KPL>& G) {
+  const uint32_t magic = la.magic;
+  const HeaCellSite c =
+      hea_cell_site<LT>(G.i, la.edge, [magic](uint32_t n) { return hea_cell_div(n, magic); });
+  int f[3][5];
+  hea_axis_terms<LT, 0>(c.c[0], c.p[0], la.edge, f[0]);
+  hea_axis_terms<LT, 1>(c.c[1], c.p[1], la.edge, f[1]);
+  hea_axis_terms<LT, 2>(c.c[2], c.p[2], la.edge, f[2]);
+  G.own();
+  gather_shell<LT, 0>(f, G);
+  if (P.S > 1) gather_shell<LT, 1>(f, G);
+  if (P.S > 2) gather_shell<LT, 2>(f, G);
+}
+template <int LT, typename T, int V, int KPL>
+__device__ __forceinline__ void gather_part(const HeaConst& P, const int32_t* nbrT,
+                                            HeaLatticeArg la, const GatherLane<T, V, KPL>& G) {
+  if constexpr (LT == HEA_LT_NONE)
+    gather_table(P, TableNbrs{nbrT, P.N, G.i, nullptr}, G);
+  else
+    gather_stencil<LT>(P, la, G);
 }
 
 // Q[s][i][c] for one block of SB sites, then the block's share of
@@ -162,10 +251,10 @@ __device__ __forceinline__ void gather_part(const HeaConst& P, const int32_t* __
 // part B (W2 > 0) the first half of the workgroup's waves gathers part A
 // of SB = 256 sites and the second half part B of the same sites, so every
 // wave loads rows of one width.  LDS rows are KPL = 4 or 8 columns wide.
-template <typename T, int W2>
+template <typename T, int W2, int LT>
 __global__ __launch_bounds__(kGatherThreads) void k_gather_pairs(
-    const HeaConst* __restrict__ pc, const int32_t* __restrict__ nbrT, const T* __restrict__ pp,
-    T* __restrict__ Q, double* __restrict__ part) {
+    const HeaConst* __restrict__ pc, const int32_t* __restrict__ nbrT, HeaLatticeArg la,
+    const T* __restrict__ pp, T* __restrict__ Q, double* __restrict__ part) {
   constexpr int G = W2 > 0 ? 2 : 1, SB = kGatherThreads / G, KPL = 4 * G;
   __shared__ T sp[SB * KPL];
   __shared__ T sq[HEA_MAX_S * SB * KPL];
@@ -177,10 +266,11 @@ __global__ __launch_bounds__(kGatherThreads) void k_gather_pairs(
   const int i = blk * SB + il;
   if (i < N) {
     if (b == 0)
-      gather_part<T, 4, KPL>(P, nbrT, pp, Q, i, SB, il, 0, sp, sq);
+      gather_part<LT>(P, nbrT, la, GatherLane<T, 4, KPL>{pp, Q, N, SB, i, il, 0, sp, sq});
     else if constexpr (W2 > 0)
-      gather_part<T, W2, KPL>(P, nbrT, pp + (size_t)4 * N, Q + (size_t)4 * S * N, i, SB, il, 4,
-                              sp, sq);
+      gather_part<LT>(P, nbrT, la,
+                      GatherLane<T, W2, KPL>{pp + (size_t)4 * N, Q + (size_t)4 * S * N, N, SB, i,
+                                             il, 4, sp, sq});
   }
   // zeros for absent sites and the padding columns the pair sums never read
   // beyond K; every LDS column of a present site is written above or here
@@ -206,19 +296,63 @@ __global__ __launch_bounds__(kGatherThreads) void k_gather_pairs(
 
 // n[e] = sum over the nb block partials of entry e: strided lane sums, then
 // a fixed-shape tree (one workgroup per entry).
-__global__ __launch_bounds__(256) void k_pair_reduce(const double* __restrict__ part, int nb,
-                                                     double* __restrict__ n) {
-  __shared__ double r[256];
-  const double* row = part + (size_t)blockIdx.x * nb;
-  double acc = 0.0;
-  for (int x = threadIdx.x; x < nb; x += 256) acc += row[x];
-  r[threadIdx.x] = acc;
+__device__ __forceinline__ double reduce_tree(double* r, double v) {
+  r[threadIdx.x] = v;
   __syncthreads();
   for (int w = 128; w > 0; w >>= 1) {
     if ((int)threadIdx.x < w) r[threadIdx.x] += r[threadIdx.x + w];
     __syncthreads();
   }
-  if (threadIdx.x == 0) n[blockIdx.x] = r[0];
+  return r[0];
+}
+__device__ __forceinline__ double reduce_entry(const double* __restrict__ part, int nb,
+                                               double* r) {
+  const double* row = part + (size_t)blockIdx.x * nb;
+  double acc = 0.0;
+  for (int x = threadIdx.x; x < nb; x += 256) acc += row[x];
+  return reduce_tree(r, acc);
+}
+__global__ __launch_bounds__(256) void k_pair_reduce(const double* __restrict__ part, int nb,
+                                                     double* __restrict__ n) {
+  __shared__ double r[256];
+  const double v = reduce_entry(part, nb, r);
+  if (threadIdx.x == 0) n[blockIdx.x] = v;
+}
+
+// k_pair_reduce, and in the last workgroup to finish the relaxed objective
+//   F^2 = sum_s w_s sum_ab d_sab^2,  d = 1 - (n / zn_s) / cc_ab - t_sab,
+// and dF^2/dn = -2 w_s d / (zn_s cc_ab): the K x K algebra of a dozen tensor
+// operations each way (a step of 4000 to 500000 sites took 250 us, most of it
+// their launches, and takes 64 to 130) costs no launch of its own: 5.0-7.9 us,
+// 3.9-4.6 of them k_pair_reduce's.  n is exchanged with agent scope (the workgroups may sit on
+// different XCDs); ticket wraps to 0 by itself.
+__global__ __launch_bounds__(256) void k_pair_objective(
+    const double* __restrict__ part, int nb, double* n, int S, int KK,
+    const double* __restrict__ zn, const double* __restrict__ cc,
+    const double* __restrict__ target, const double* __restrict__ weight, uint32_t* ticket,
+    double* __restrict__ f2, double* __restrict__ dn) {
+  __shared__ double r[256];
+  __shared__ uint32_t last;
+  const double v = reduce_entry(part, nb, r);
+  if (threadIdx.x == 0) {
+    __hip_atomic_store(n + blockIdx.x, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __threadfence();
+    last = atomicInc(ticket, gridDim.x - 1) == gridDim.x - 1;
+  }
+  __syncthreads();
+  if (!last) return;
+  __threadfence();
+  double term = 0.0;
+  const int e = threadIdx.x;  // S K K <= 192 entries
+  if (e < S * KK) {
+    const int s = e / KK, ab = e - s * KK;
+    const double ne = __hip_atomic_load(n + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const double d = 1.0 - (ne / zn[s]) / cc[ab] - target[e];
+    term = weight[s] * (d * d);
+    dn[e] = -2.0 * weight[s] * d / (zn[s] * cc[ab]);
+  }
+  const double sum = reduce_tree(r, term);
+  if (threadIdx.x == 0) *f2 = sum;
 }
 
 // grad[k][c] = p[k][c] (g[k][c] - sum_d p[k][d] g[k][d]),
@@ -232,6 +366,7 @@ __global__ __launch_bounds__(256) void k_adjoint(const HeaConst* __restrict__ pc
                                                  const T* __restrict__ p,
                                                  const T* __restrict__ Q,
                                                  const double* __restrict__ dn,
+                                                 const double* __restrict__ scale,
                                                  T* __restrict__ grad) {
   constexpr int GL = W2 > 0 ? 2 : 1, C = 4 + W2;
   using VA = VecT<T, 4>;
@@ -265,9 +400,10 @@ __global__ __launch_bounds__(256) void k_adjoint(const HeaConst* __restrict__ pc
       for (int v = 0; v < W2; ++v) pr[4 + v] = pb.x[v];
     }
   }
+  const double sc = scale ? *scale : 1.0;  // d loss / d F^2 where dn is dF^2/dn
   for (int e = threadIdx.x; e < S * K * K; e += blockDim.x) {
     const int s = e / (K * K), c = (e / K) % K, bb = e % K;
-    H[e] = dn[(s * K + c) * K + bb] + dn[(s * K + bb) * K + c];
+    H[e] = sc * (dn[(s * K + c) * K + bb] + dn[(s * K + bb) * K + c]);
   }
   __syncthreads();
   if (!live) return;
@@ -334,26 +470,43 @@ inline int relax_gather_blocks(int N, int K) {
   return (N + sb - 1) / sb;
 }
 
+template <typename T, int W2, int LT>
+void launch_gather(const HeaConst* dc, const HeaConst& hc, const int32_t* nbrT, HeaLatticeArg la,
+                   const T* p, T* Q, double* part, hipStream_t st) {
+  hipLaunchKernelGGL((k_gather_pairs<T, W2, LT>), dim3(relax_gather_blocks(hc.N, hc.K)),
+                     dim3(kGatherThreads), 0, st, dc, nbrT, la, p, Q, part);
+}
+
 template <typename T, int W2>
 hipError_t relax_forward_g(const HeaConst* dc, const HeaConst& hc, const int32_t* nbrT,
-                           const void* th, void* p, void* Q, double* part, double* n,
-                           hipStream_t st) {
+                           HeaLatticeArg la, const void* th, void* p, void* Q, double* part,
+                           double* n, const HeaObjectiveArg* ob, hipStream_t st) {
+  T *pt = static_cast<T*>(p), *qt = static_cast<T*>(Q);
   hipLaunchKernelGGL((k_softmax<T, W2>), dim3((hc.N + kSoftmaxThreads - 1) / kSoftmaxThreads),
-                     dim3(kSoftmaxThreads), 0, st, static_cast<const T*>(th), static_cast<T*>(p),
-                     hc.N, hc.K);
-  const int nb = relax_gather_blocks(hc.N, hc.K);
-  hipLaunchKernelGGL((k_gather_pairs<T, W2>), dim3(nb), dim3(kGatherThreads), 0, st, dc, nbrT,
-                     static_cast<const T*>(p), static_cast<T*>(Q), part);
-  hipLaunchKernelGGL(k_pair_reduce, dim3(hc.S * hc.K * hc.K), dim3(256), 0, st, part, nb, n);
+                     dim3(kSoftmaxThreads), 0, st, static_cast<const T*>(th), pt, hc.N, hc.K);
+  switch (la.lt) {
+    case HEA_LT_FCC: launch_gather<T, W2, HEA_LT_FCC>(dc, hc, nbrT, la, pt, qt, part, st); break;
+    case HEA_LT_FCC_REF:
+      launch_gather<T, W2, HEA_LT_FCC_REF>(dc, hc, nbrT, la, pt, qt, part, st);
+      break;
+    case HEA_LT_BCC: launch_gather<T, W2, HEA_LT_BCC>(dc, hc, nbrT, la, pt, qt, part, st); break;
+    default: launch_gather<T, W2, HEA_LT_NONE>(dc, hc, nbrT, la, pt, qt, part, st);
+  }
+  const int nb = relax_gather_blocks(hc.N, hc.K), KK = hc.K * hc.K;
+  if (ob)
+    hipLaunchKernelGGL(k_pair_objective, dim3(hc.S * KK), dim3(256), 0, st, part, nb, n, hc.S, KK,
+                       ob->zn, ob->cc, ob->target, ob->weight, ob->ticket, ob->f2, ob->dn);
+  else
+    hipLaunchKernelGGL(k_pair_reduce, dim3(hc.S * KK), dim3(256), 0, st, part, nb, n);
   return hipGetLastError();
 }
 
 template <typename T, int W2>
 hipError_t relax_backward_t(const HeaConst* dc, const HeaConst& hc, const void* p, const void* Q,
-                            const double* dn, void* grad, hipStream_t st) {
+                            const double* dn, const double* scale, void* grad, hipStream_t st) {
   const int lanes = hc.N * (W2 > 0 ? 2 : 1);
   hipLaunchKernelGGL((k_adjoint<T, W2>), dim3((lanes + 255) / 256), dim3(256), 0, st, dc,
-                     static_cast<const T*>(p), static_cast<const T*>(Q), dn,
+                     static_cast<const T*>(p), static_cast<const T*>(Q), dn, scale,
                      static_cast<T*>(grad));
   return hipGetLastError();
 }
@@ -381,17 +534,17 @@ hipError_t relax_dispatch(int dtype, int K, Args... args) {
 template <typename T, int W2>
 struct RelaxForward {
   static hipError_t run(const HeaConst* dc, const HeaConst* hc, const int32_t* nbrT,
-                        const void* th, void* p, void* Q, double* part, double* n,
-                        hipStream_t st) {
-    return relax_forward_g<T, W2>(dc, *hc, nbrT, th, p, Q, part, n, st);
+                        HeaLatticeArg la, const void* th, void* p, void* Q, double* part, double* n,
+                        const HeaObjectiveArg* ob, hipStream_t st) {
+    return relax_forward_g<T, W2>(dc, *hc, nbrT, la, th, p, Q, part, n, ob, st);
   }
 };
 
 template <typename T, int W2>
 struct RelaxBackward {
   static hipError_t run(const HeaConst* dc, const HeaConst* hc, const void* p, const void* Q,
-                        const double* dn, void* grad, hipStream_t st) {
-    return relax_backward_t<T, W2>(dc, *hc, p, Q, dn, grad, st);
+                        const double* dn, const double* scale, void* grad, hipStream_t st) {
+    return relax_backward_t<T, W2>(dc, *hc, p, Q, dn, scale, grad, st);
   }
 };
 
@@ -414,15 +567,16 @@ hipError_t hea_relax_transpose_nbr(const int32_t* nbr, int N, int stride, int32_
 }
 
 hipError_t hea_relax_forward_impl(const HeaConst* dc, const HeaConst& hc, const int32_t* nbrT,
-                                  int dtype, const void* th, void* p, void* Q, double* part,
-                                  double* n, hipStream_t st) {
-  return relax_dispatch<RelaxForward>(dtype, hc.K, dc, &hc, nbrT, th, p, Q, part, n, st);
+                                  HeaLatticeArg la, int dtype, const void* th, void* p, void* Q,
+                                  double* part, double* n, const HeaObjectiveArg* ob,
+                                  hipStream_t st) {
+  return relax_dispatch<RelaxForward>(dtype, hc.K, dc, &hc, nbrT, la, th, p, Q, part, n, ob, st);
 }
 
 hipError_t hea_relax_backward_impl(const HeaConst* dc, const HeaConst& hc, int dtype,
-                                   const void* p, const void* Q, const double* dn, void* grad,
-                                   hipStream_t st) {
-  return relax_dispatch<RelaxBackward>(dtype, hc.K, dc, &hc, p, Q, dn, grad, st);
+                                   const void* p, const void* Q, const double* dn,
+                                   const double* scale, void* grad, hipStream_t st) {
+  return relax_dispatch<RelaxBackward>(dtype, hc.K, dc, &hc, p, Q, dn, scale, grad, st);
 }
 
 hipError_t hea_site_gain_impl(const HeaConst* dc, const HeaConst& hc, const int32_t* nbrT,
