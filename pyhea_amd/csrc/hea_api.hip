@@ -262,24 +262,39 @@ __device__ __forceinline__ void recount_stencil(const HeaConst& P,
     const int i = i0 + tid;
     if (i < N) {
       const HeaCellSite c = hea_cell_site<LT>(i, edge, div);
-      const SiteTerms t = site_terms<LT, false>(c, edge, spa);
       const int a = Species<false, PK::W>::species_of(sp[i]);
-      auto shell = [&](auto sc, uint32_t& h) {
-        constexpr int s = decltype(sc)::value;
-        uint32_t v[HeaShells<LT>::Z[s]];
-        load_shell<LT, s>(t, v);
-        __builtin_amdgcn_sched_barrier(0);
-        h = 0;
-        count_shell<KMAX, LT, s, false>(t, v, h);
+      auto add = [&](int s, uint32_t h) {
         unsigned long long w = 0ull;
 #pragma unroll
         for (int x = 0; x < F; ++x) w |= (unsigned long long)PK::fld(h, x) << (x * FW);
         atomicAdd(&my[s * KMAX + a], w);
       };
-      uint32_t h;
-      shell(std::integral_constant<int, 0>{}, h);
-      if (S > 1) shell(std::integral_constant<int, 1>{}, h);
-      if (S > 2) shell(std::integral_constant<int, 2>{}, h);
+      bool by_cell = false;
+      if constexpr (LT == HEA_LT_FCC || LT == HEA_LT_FCC_REF) {
+        if (S == 3) {
+          const CellTerms t = cell_terms<false>(c, edge, spa);
+          uint32_t w[27], h[HEA_MAX_S] = {};
+          load_cells<LT, false>(t, w);
+          __builtin_amdgcn_sched_barrier(0);
+          count_cells<KMAX, LT, false>(t, w, h);
+          for (int s = 0; s < HEA_MAX_S; ++s) add(s, h[s]);
+          by_cell = true;
+        }
+      }
+      if (!by_cell) {
+        const SiteTerms t = site_terms<LT, false>(c, edge, spa);
+        auto shell = [&](auto sc) {
+          constexpr int s = decltype(sc)::value;
+          uint32_t v[HeaShells<LT>::Z[s]], h = 0;
+          load_shell<LT, s>(t, v);
+          __builtin_amdgcn_sched_barrier(0);
+          count_shell<KMAX, LT, s, false>(t, v, h);
+          add(s, h);
+        };
+        shell(std::integral_constant<int, 0>{});
+        if (S > 1) shell(std::integral_constant<int, 1>{});
+        if (S > 2) shell(std::integral_constant<int, 2>{});
+      }
     }
     if (++pass == FLUSH) {
       flush();

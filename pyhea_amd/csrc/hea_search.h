@@ -165,11 +165,27 @@ __device__ __forceinline__ void walk_shell(const SiteTerms* t, typename Pack<KMA
 }
 
 template <int KMAX, int LT, bool NIB>
-__device__ __forceinline__ void walk_sites(const SiteTerms* t, int S,
-                                           typename Pack<KMAX>::T* MA,
+__device__ __forceinline__ void walk_sites(const HeaCellSite& ca, const HeaCellSite& cb, int L,
+                                           uint32_t sp, int S, typename Pack<KMAX>::T* MA,
                                            typename Pack<KMAX>::T* MB) {
 #pragma unroll
   for (int s = 0; s < HEA_MAX_S; ++s) MA[s] = MB[s] = 0;
+  if constexpr (LT == HEA_LT_FCC || LT == HEA_LT_FCC_REF) {
+    if (S == 3) {  // fewer shells: not all of the cells
+      uint32_t w[27];
+      const CellTerms ta = cell_terms<NIB>(ca, L, sp);
+      load_cells<LT, NIB>(ta, w);
+      __builtin_amdgcn_sched_barrier(0);
+      const CellTerms tb = cell_terms<NIB>(cb, L, sp);
+      uint32_t v[27];
+      load_cells<LT, NIB>(tb, v);
+      __builtin_amdgcn_sched_barrier(0);
+      count_cells<KMAX, LT, NIB>(ta, w, MA);
+      count_cells<KMAX, LT, NIB>(tb, v, MB);
+      return;
+    }
+  }
+  const SiteTerms t[2] = {site_terms<LT, NIB>(ca, L, sp), site_terms<LT, NIB>(cb, L, sp)};
   walk_shell<KMAX, LT, 0, NIB>(t, MA[0], MB[0]);
   if (S > 1) walk_shell<KMAX, LT, 1, NIB>(t, MA[1], MB[1]);
   if (S > 2) walk_shell<KMAX, LT, 2, NIB>(t, MA[2], MB[2]);
@@ -612,9 +628,7 @@ __device__ __forceinline__ SearchCounts worker_rounds(const HeaMcArgs& A,
       const uint32_t spa = lds_addr(sp.p);
       const HeaCellSite ca = hea_cell_site<LT>(pr.x, L, div);
       const HeaCellSite cb = hea_cell_site<LT>(pr.y, L, div);
-      const SiteTerms t[2] = {site_terms<LT, NIB>(ca, L, spa),
-                              site_terms<LT, NIB>(cb, L, spa)};
-      walk_sites<KMAX, LT, NIB>(t, S, MA, MB);
+      walk_sites<KMAX, LT, NIB>(ca, cb, L, spa, S, MA, MB);
       d2 = hea_cell_dist2(ca, cb, L);
     }
     const int a = SP::species_of(sa), b = SP::species_of(sb);

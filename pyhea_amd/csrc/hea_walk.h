@@ -2,6 +2,8 @@
 // neighbours' ids from its coordinates (hea_stencil.h), their species gathered
 // from LDS, and the shells' species histograms.
 #pragma once
+#include <type_traits>
+
 #include "hea_exact.h"
 #include "hea_screen.h"
 #include "hea_stencil.h"
@@ -44,6 +46,10 @@ __device__ __forceinline__ void count_species(uint32_t& m, uint32_t s) {
   asm("v_lshl_add_u32 %0, 1, %1, %0" : "+v"(m) : "v"(s));
 }
 __device__ __forceinline__ void count_species(uint64_t& m, uint32_t s) { m += 1ull << s; }
+// The same for a shift in the low byte of s: the instruction takes the low five
+// (six) bits, and the shifts of species stay below.
+__device__ __forceinline__ void count_species_low(uint32_t& m, uint32_t s) { count_species(m, s); }
+__device__ __forceinline__ void count_species_low(uint64_t& m, uint32_t s) { m += 1ull << (s & 63u); }
 
 // x + y + z in one instruction (left to itself the compiler shares pair sums
 // and needs half as many again).
@@ -110,6 +116,93 @@ __device__ __forceinline__ void count_shell(const SiteTerms& t, const uint32_t* 
           }
           count_species(m, x);
         }
+}
+
+// ---- walks by cell: both FCC shell sets, with three shells ----
+//
+// The four sites of a cell are the four bytes (or nibbles) of one LDS word, and
+// the 42 (30) neighbours of a site lie in 20 (19) cells: one load per cell
+// instead of one per neighbour, and one instruction more per neighbour.  The walk
+// is bound by LDS: bytes at random addresses, 6 to 7 cycles a load with their
+// bank conflicts, kept it busy 56 % of a search of 108000 sites.  That search
+// takes 95.6 ms, 106.5 by neighbour (512 proposals a round); 256000 sites two a
+// byte 214.8, 232.0; 4000 sites of 30 neighbours 3.54, 3.65.  BCC's 26
+// neighbours lie in 20 cells of two sites, which gains nothing.
+// Seen from a site of odd parity on an axis the cells are
+// mirrored on it, so with k the mirrored cell of a (mirrored) step d,
+//     k = -1, -1, 0, 0, 1 for d = -2 .. 2,
+// every lane needs the same cells; the neighbour is site b ^ m of its cell, b the
+// site's own number and m the parities of the step.
+struct CellTerms {
+  uint32_t g[3][3];  // address terms of cells -1, 0, 1 (mirrored) on each axis
+  uint32_t sh[4];    // bit of site b ^ m in its cell's word
+};
+__host__ __device__ constexpr int step_cell(int d) { return d < 0 ? -1 : d > 1 ? 1 : 0; }
+// Whether a shell of LT has a neighbour in cell (x, y, z).
+template <int LT>
+__host__ __device__ constexpr bool cell_used(int x, int y, int z) {
+  for (int dx = -2; dx <= 2; ++dx)
+    for (int dy = -2; dy <= 2; ++dy)
+      for (int dz = -2; dz <= 2; ++dz)
+        if (HeaShells<LT>::shell(dx, dy, dz) >= 0 && step_cell(dx) == x && step_cell(dy) == y &&
+            step_cell(dz) == z)
+          return true;
+  return false;
+}
+template <bool NIB>
+__device__ __forceinline__ CellTerms cell_terms(const HeaCellSite& c, int L, uint32_t sp) {
+  constexpr int CB = NIB ? 2 : 4;  // bytes of a cell
+  CellTerms t;
+#pragma unroll
+  for (int x = 0; x < 3; ++x) {
+    const int A = x == 0 ? CB * L * L : x == 1 ? CB * L : CB;
+    const int at = hea_mul24(A, c.c[x]), span = A * (L - 1);
+    const int up = c.c[x] == L - 1 ? at - span : at + A;
+    const int dn = c.c[x] == 0 ? at + span : at - A;
+    t.g[x][0] = (uint32_t)(c.p[x] ? up : dn);
+    t.g[x][1] = (uint32_t)at;
+    t.g[x][2] = (uint32_t)(c.p[x] ? dn : up);
+  }
+#pragma unroll
+  for (int k = 0; k < 3; ++k) t.g[0][k] += sp;
+  constexpr uint32_t B = NIB ? 4 : 8;  // bits of a site
+  t.sh[0] = B * (uint32_t)(c.p[1] | (c.p[2] << 1));
+#pragma unroll
+  for (uint32_t m = 1; m < 4; ++m) t.sh[m] = t.sh[0] ^ (B * m);
+  return t;
+}
+template <int LT, bool NIB>
+__device__ __forceinline__ void load_cells(const CellTerms& t, uint32_t* w) {
+  using Word = std::conditional_t<NIB, const __attribute__((address_space(3))) uint16_t,
+                                  const __attribute__((address_space(3))) uint32_t>;
+#pragma unroll
+  for (int x = 0; x < 3; ++x)
+#pragma unroll
+    for (int y = 0; y < 3; ++y)
+#pragma unroll
+      for (int z = 0; z < 3; ++z)
+        if (cell_used<LT>(x - 1, y - 1, z - 1))
+          w[(x * 3 + y) * 3 + z] = *(Word*)(uintptr_t)add3(t.g[0][x], t.g[1][y], t.g[2][z]);
+}
+template <int KMAX, int LT, bool NIB>
+__device__ __forceinline__ void count_cells(const CellTerms& t, const uint32_t* w,
+                                            typename Pack<KMAX>::T* m) {
+#pragma unroll
+  for (int dx = -2; dx <= 2; ++dx)
+#pragma unroll
+    for (int dy = -2; dy <= 2; ++dy)
+#pragma unroll
+      for (int dz = -2; dz <= 2; ++dz) {
+        const int s = HeaShells<LT>::shell(dx, dy, dz);
+        if (s >= 0) {
+          const uint32_t c = w[((step_cell(dx) + 1) * 3 + step_cell(dy) + 1) * 3 + step_cell(dz) + 1];
+          const uint32_t bit = t.sh[(dy & 1) | ((dz & 1) << 1)];
+          if constexpr (NIB)
+            count_species(m[s], (uint32_t)Pack<KMAX>::W * __builtin_amdgcn_ubfe(c, bit, 4));
+          else
+            count_species_low(m[s], c >> bit);
+        }
+      }
 }
 
 }  // namespace

@@ -85,3 +85,10 @@ def test_two_species_a_byte_equals_the_hbm_walk(gpu, monkeypatch, latt, edge, sh
     b = q.local_mc(lat, fit, task, 3, seed=6)
     assert np.array_equal(a[0], b[0]) and np.array_equal(_bits(a[1]), _bits(b[1]))
     assert all(a[2][c] == b[2][c] for c in ("evals", "rounds", "accepts", "draws"))
+
+
+@pytest.mark.parametrize("edge,shells,k", [(3, "pyhea", 4), (4, "true", 6), (4, "true", 7),
+                                           (5, "pyhea", 6), (6, "true", 4), (7, "pyhea", 8)])
+def test_walks_by_cell(gpu, edge, shells, k):
+    """Each parity of the edge and each width of the histograms."""
+    _check(make_problem("FCC", edge, np.arange(2, k + 2), shells=shells, target_seed=k), 100, 3)
