@@ -269,32 +269,30 @@ __device__ __forceinline__ void recount_stencil(const HeaConst& P,
         for (int x = 0; x < F; ++x) w |= (unsigned long long)PK::fld(h, x) << (x * FW);
         atomicAdd(&my[s * KMAX + a], w);
       };
-      bool by_cell = false;
+      uint32_t h[HEA_MAX_S] = {};
       if constexpr (LT == HEA_LT_FCC || LT == HEA_LT_FCC_REF) {
-        if (S == 3) {
-          const CellTerms t = cell_terms<false>(c, edge, spa);
-          uint32_t w[27], h[HEA_MAX_S] = {};
-          load_cells<LT, false>(t, w);
-          __builtin_amdgcn_sched_barrier(0);
-          count_cells<KMAX, LT, false>(t, w, h);
-          for (int s = 0; s < HEA_MAX_S; ++s) add(s, h[s]);
-          by_cell = true;
-        }
-      }
-      if (!by_cell) {
+        if (S == 3)
+          walk_cells<KMAX, LT, 3, false>(c, edge, spa, h);
+        else if (S == 2)
+          walk_cells<KMAX, LT, 2, false>(c, edge, spa, h);
+        else
+          walk_cells<KMAX, LT, 1, false>(c, edge, spa, h);
+      } else {
         const SiteTerms t = site_terms<LT, false>(c, edge, spa);
         auto shell = [&](auto sc) {
           constexpr int s = decltype(sc)::value;
-          uint32_t v[HeaShells<LT>::Z[s]], h = 0;
+          uint32_t v[HeaShells<LT>::Z[s]];
           load_shell<LT, s>(t, v);
           __builtin_amdgcn_sched_barrier(0);
-          count_shell<KMAX, LT, s, false>(t, v, h);
-          add(s, h);
+          count_shell<KMAX, LT, s, false>(t, v, h[s]);
         };
         shell(std::integral_constant<int, 0>{});
         if (S > 1) shell(std::integral_constant<int, 1>{});
         if (S > 2) shell(std::integral_constant<int, 2>{});
       }
+      add(0, h[0]);
+      if (S > 1) add(1, h[1]);
+      if (S > 2) add(2, h[2]);
     }
     if (++pass == FLUSH) {
       flush();

@@ -164,6 +164,22 @@ __device__ __forceinline__ void walk_shell(const SiteTerms* t, typename Pack<KMA
   count_shell<KMAX, LT, SHELL, NIB>(t[1], vb, mb);
 }
 
+// The same by cell (both sites' loads are under way before the first count).
+template <int KMAX, int LT, int NS, bool NIB>
+__device__ __forceinline__ void walk_pair(const HeaCellSite& ca, const HeaCellSite& cb, int L,
+                                          uint32_t sp, typename Pack<KMAX>::T* MA,
+                                          typename Pack<KMAX>::T* MB) {
+  uint32_t va[27], vb[27];
+  const CellTerms ta = cell_terms<NIB>(ca, L, sp);
+  load_cells<LT, NS, NIB>(ta, va);
+  __builtin_amdgcn_sched_barrier(0);
+  const CellTerms tb = cell_terms<NIB>(cb, L, sp);
+  load_cells<LT, NS, NIB>(tb, vb);
+  __builtin_amdgcn_sched_barrier(0);
+  count_cells<KMAX, LT, NS, NIB>(ta, va, MA);
+  count_cells<KMAX, LT, NS, NIB>(tb, vb, MB);
+}
+
 template <int KMAX, int LT, bool NIB>
 __device__ __forceinline__ void walk_sites(const HeaCellSite& ca, const HeaCellSite& cb, int L,
                                            uint32_t sp, int S, typename Pack<KMAX>::T* MA,
@@ -171,24 +187,18 @@ __device__ __forceinline__ void walk_sites(const HeaCellSite& ca, const HeaCellS
 #pragma unroll
   for (int s = 0; s < HEA_MAX_S; ++s) MA[s] = MB[s] = 0;
   if constexpr (LT == HEA_LT_FCC || LT == HEA_LT_FCC_REF) {
-    if (S == 3) {  // fewer shells: not all of the cells
-      uint32_t w[27];
-      const CellTerms ta = cell_terms<NIB>(ca, L, sp);
-      load_cells<LT, NIB>(ta, w);
-      __builtin_amdgcn_sched_barrier(0);
-      const CellTerms tb = cell_terms<NIB>(cb, L, sp);
-      uint32_t v[27];
-      load_cells<LT, NIB>(tb, v);
-      __builtin_amdgcn_sched_barrier(0);
-      count_cells<KMAX, LT, NIB>(ta, w, MA);
-      count_cells<KMAX, LT, NIB>(tb, v, MB);
-      return;
-    }
+    if (S == 3)
+      walk_pair<KMAX, LT, 3, NIB>(ca, cb, L, sp, MA, MB);
+    else if (S == 2)
+      walk_pair<KMAX, LT, 2, NIB>(ca, cb, L, sp, MA, MB);
+    else
+      walk_pair<KMAX, LT, 1, NIB>(ca, cb, L, sp, MA, MB);
+  } else {
+    const SiteTerms t[2] = {site_terms<LT, NIB>(ca, L, sp), site_terms<LT, NIB>(cb, L, sp)};
+    walk_shell<KMAX, LT, 0, NIB>(t, MA[0], MB[0]);
+    if (S > 1) walk_shell<KMAX, LT, 1, NIB>(t, MA[1], MB[1]);
+    if (S > 2) walk_shell<KMAX, LT, 2, NIB>(t, MA[2], MB[2]);
   }
-  const SiteTerms t[2] = {site_terms<LT, NIB>(ca, L, sp), site_terms<LT, NIB>(cb, L, sp)};
-  walk_shell<KMAX, LT, 0, NIB>(t, MA[0], MB[0]);
-  if (S > 1) walk_shell<KMAX, LT, 1, NIB>(t, MA[1], MB[1]);
-  if (S > 2) walk_shell<KMAX, LT, 2, NIB>(t, MA[2], MB[2]);
 }
 
 template <int CTRL, int ROWS>

@@ -118,10 +118,11 @@ __device__ __forceinline__ void count_shell(const SiteTerms& t, const uint32_t* 
         }
 }
 
-// ---- walks by cell: both FCC shell sets, with three shells ----
+// ---- walks by cell: both FCC shell sets ----
 //
 // The four sites of a cell are the four bytes (or nibbles) of one LDS word, and
-// the 42 (30) neighbours of a site lie in 20 (19) cells: one load per cell
+// the 42 (30) neighbours of a site lie in 20 (19) cells, those of the first two
+// shells, 18, in 10 and the first's 12 in 7: one load per cell
 // instead of one per neighbour, and one instruction more per neighbour.  The walk
 // is bound by LDS: bytes at random addresses, 6 to 7 cycles a load with their
 // bank conflicts, kept it busy 56 % of a search of 108000 sites.  That search
@@ -138,14 +139,14 @@ struct CellTerms {
   uint32_t sh[4];    // bit of site b ^ m in its cell's word
 };
 __host__ __device__ constexpr int step_cell(int d) { return d < 0 ? -1 : d > 1 ? 1 : 0; }
-// Whether a shell of LT has a neighbour in cell (x, y, z).
-template <int LT>
+// Whether one of LT's first NS shells has a neighbour in cell (x, y, z).
+template <int LT, int NS>
 __host__ __device__ constexpr bool cell_used(int x, int y, int z) {
   for (int dx = -2; dx <= 2; ++dx)
     for (int dy = -2; dy <= 2; ++dy)
       for (int dz = -2; dz <= 2; ++dz)
-        if (HeaShells<LT>::shell(dx, dy, dz) >= 0 && step_cell(dx) == x && step_cell(dy) == y &&
-            step_cell(dz) == z)
+        if (HeaShells<LT>::shell(dx, dy, dz) >= 0 && HeaShells<LT>::shell(dx, dy, dz) < NS &&
+            step_cell(dx) == x && step_cell(dy) == y && step_cell(dz) == z)
           return true;
   return false;
 }
@@ -171,7 +172,7 @@ __device__ __forceinline__ CellTerms cell_terms(const HeaCellSite& c, int L, uin
   for (uint32_t m = 1; m < 4; ++m) t.sh[m] = t.sh[0] ^ (B * m);
   return t;
 }
-template <int LT, bool NIB>
+template <int LT, int NS, bool NIB>
 __device__ __forceinline__ void load_cells(const CellTerms& t, uint32_t* w) {
   using Word = std::conditional_t<NIB, const __attribute__((address_space(3))) uint16_t,
                                   const __attribute__((address_space(3))) uint32_t>;
@@ -181,10 +182,10 @@ __device__ __forceinline__ void load_cells(const CellTerms& t, uint32_t* w) {
     for (int y = 0; y < 3; ++y)
 #pragma unroll
       for (int z = 0; z < 3; ++z)
-        if (cell_used<LT>(x - 1, y - 1, z - 1))
+        if (cell_used<LT, NS>(x - 1, y - 1, z - 1))
           w[(x * 3 + y) * 3 + z] = *(Word*)(uintptr_t)add3(t.g[0][x], t.g[1][y], t.g[2][z]);
 }
-template <int KMAX, int LT, bool NIB>
+template <int KMAX, int LT, int NS, bool NIB>
 __device__ __forceinline__ void count_cells(const CellTerms& t, const uint32_t* w,
                                             typename Pack<KMAX>::T* m) {
 #pragma unroll
@@ -194,7 +195,7 @@ __device__ __forceinline__ void count_cells(const CellTerms& t, const uint32_t* 
 #pragma unroll
       for (int dz = -2; dz <= 2; ++dz) {
         const int s = HeaShells<LT>::shell(dx, dy, dz);
-        if (s >= 0) {
+        if (s >= 0 && s < NS) {
           const uint32_t c = w[((step_cell(dx) + 1) * 3 + step_cell(dy) + 1) * 3 + step_cell(dz) + 1];
           const uint32_t bit = t.sh[(dy & 1) | ((dz & 1) << 1)];
           if constexpr (NIB)
@@ -203,6 +204,17 @@ __device__ __forceinline__ void count_cells(const CellTerms& t, const uint32_t* 
             count_species_low(m[s], c >> bit);
         }
       }
+}
+
+// Species histograms m of a site's first NS shells.
+template <int KMAX, int LT, int NS, bool NIB>
+__device__ __forceinline__ void walk_cells(const HeaCellSite& c, int L, uint32_t sp,
+                                           typename Pack<KMAX>::T* m) {
+  const CellTerms t = cell_terms<NIB>(c, L, sp);
+  uint32_t w[27];
+  load_cells<LT, NS, NIB>(t, w);
+  __builtin_amdgcn_sched_barrier(0);
+  count_cells<KMAX, LT, NS, NIB>(t, w, m);
 }
 
 }  // namespace
