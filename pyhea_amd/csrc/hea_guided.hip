@@ -30,6 +30,7 @@
 //
 // Barriers of a round: BD difference table ready; B1 minima published; BS
 // shortlist ready (accepts only); BA accepts done.
+#include <algorithm>
 #include <type_traits>
 #include <utility>
 
@@ -223,13 +224,117 @@ __device__ __forceinline__ uint2 load_rec(const unsigned long long* rec, uint32_
   }
 }
 
+// What an accepted swap (v.x: species v.z -> v.w, v.y: back) changes besides the
+// tables: its sites' neighbours' records, and the round's maps.  By all lanes of
+// one wave.
+template <int KMAX, int LT, bool RL>
+__device__ __forceinline__ void touch(const GuidedTab<KMAX, RL>& T, unsigned long long* rec,
+                                      const int4& v, int L, int blk, float inv_edge, int lane) {
+  constexpr int K = KMAX;
+  constexpr int ZS = HeaShells<LT>::Z[0] + HeaShells<LT>::Z[1] + HeaShells<LT>::Z[2];
+  const auto div = [inv_edge](uint32_t x) { return hea_cell_div_small(x, inv_edge); };
+  // items lane and lane + 64 of [0, 2 Z): a neighbour of s1, then of s2
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int t = opaque(lane) + 64 * u;
+    const bool one = t < ZS, on = t < 2 * ZS;
+    const int vec = T.vec[on ? (one ? t : t - ZS) : 0];
+    const HeaCellSite c = hea_cell_site<LT>(one ? v.x : v.y, L, div);
+    int id = 0;
+#pragma unroll
+    for (int x = 0; x < 3; ++x) {
+      int V = 2 * c.c[x] + c.p[x] + ((vec >> (3 * x)) & 7) - 2;
+      V = V < 0 ? V + 2 * L : V >= 2 * L ? V - 2 * L : V;
+      using ST = HeaShells<LT>;
+      const int Bx = ST::BCC ? (x == 2) : x;
+      const int Ax = x == 0 ? ST::NB * L * L : x == 1 ? ST::NB * L : ST::NB;
+      id += hea_mul24(Ax, V >> 1) + Bx * (V & 1);
+    }
+    const int s = vec >> 9;
+    const int os = s == 0 ? RecBits<LT>::o(0) : s == 1 ? RecBits<LT>::o(1) : RecBits<LT>::o(2);
+    // the last species has no field (its count is implied)
+    const unsigned long long fa = v.z < K - 1 ? 1ull << (v.z * RecBits<LT>::W + os) : 0ull;
+    const unsigned long long fb = v.w < K - 1 ? 1ull << (v.w * RecBits<LT>::W + os) : 0ull;
+    const unsigned long long dv = one ? fb - fa : fa - fb;  // modulo 2^64
+    if (on) {
+      if constexpr (RL)
+        atomicAdd(rec + id, dv);
+      else
+        __hip_atomic_fetch_add(rec + id, dv, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      const uint32_t mb = cmap_bit(id);
+      atomicOr(&T.cmap[mb >> 5], 1u << (mb & 31u));
+      if (!RL) atomicOr(&T.bmap[(uint32_t)id >> (blk + 5)], 1u << (((uint32_t)id >> blk) & 31u));
+    }
+  }
+  if (lane < 2) {
+    const uint32_t mb = cmap_bit(lane == 0 ? v.x : v.y);
+    atomicOr(&T.cmap[mb >> 5], 1u << (mb & 31u));
+  }
+}
+
+// The helper wave takes one command at a time from the service wave: the swap
+// of touch, or v.x < 0 at the end of a round's accepts.  Both count them; a wait
+// ends because the service wave posts the end before it leaves a round and the
+// helper answers every swap.  They sit behind the stencil's vectors (at most 42).
+constexpr int kCmdSeq = 48, kCmdDone = 49, kCmd = 52;
+__device__ __forceinline__ void await(const int* at, int seq) {
+  while (__hip_atomic_load(at, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) != seq)
+    __builtin_amdgcn_s_sleep(1);
+}
+
+// Rounds of the helper wave: touch of every accepted swap, while the service
+// wave forms its rows and tables.
+template <int KMAX, int LT, bool RL>
+__device__ __forceinline__ void guided_helper(const HeaMcArgs& A, const GuidedTab<KMAX, RL>& T,
+                                              unsigned long long* rec, int nw, int lane) {
+  SearchShared* sh = T.sh;
+  const int depth = A.depth, multi = A.g_multi, L = A.edge, blk = A.g_blk;
+  const double thr = A.thr;
+  const float inv_edge = A.inv_edge;
+  int seq = 0;
+  auto serve = [&]() {
+    await(T.vec + kCmdSeq, ++seq);
+    const int4 v = *reinterpret_cast<const int4*>(T.vec + kCmd);
+    if (__builtin_amdgcn_readfirstlane(v.x) < 0) return false;
+    touch<KMAX, LT, RL>(T, rec, v, L, blk, inv_edge, lane);
+    if (lane == 0)
+      __hip_atomic_store(T.vec + kCmdDone, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+    return true;
+  };
+  __builtin_amdgcn_s_setprio(2);
+  for (int acc = 0; acc < depth;) {
+    __syncthreads();  // BD
+    const double beta = round_window(sh);
+    __syncthreads();  // B1
+    int kind = decide(sh, nw, beta, thr, lane).kind;
+    if (__builtin_expect(kind < 0, 0)) {
+      __syncthreads();
+      __syncthreads();
+      kind = __builtin_amdgcn_readfirstlane(sh->res_kind);
+    }
+    if (kind == 0) {
+      ++acc;
+    } else {
+      acc = 0;
+      serve();
+      if (multi > 1) {
+        __syncthreads();  // BS
+        while (serve()) {
+        }
+      }
+    }
+    __syncthreads();  // BA
+  }
+}
+
 // Rounds of the service wave: the accepts.
 template <int KMAX, int LT, bool RL>
 __device__ __forceinline__ void guided_service(const HeaMcArgs& A, const GuidedTab<KMAX, RL>& T,
-                                               unsigned long long* rec, int l, int nw, int lane) {
+                                               unsigned long long* rec, int l, int nw, bool help,
+                                               int lane) {
   using PK = Pack<KMAX>;
   using PT = uint32_t;
-  constexpr int K = KMAX, S = 3, Zs = HeaShells<LT>::Z[0] + HeaShells<LT>::Z[1] + HeaShells<LT>::Z[2];
+  constexpr int K = KMAX, S = 3;
   SearchShared* sh = T.sh;
   const ShellArgs& SA = sh->args;
   const int task = A.task, stride = A.stride, depth = A.depth, n = A.N, L = A.edge, blk = A.g_blk;
@@ -237,7 +342,14 @@ __device__ __forceinline__ void guided_service(const HeaMcArgs& A, const GuidedT
   const double thr = A.thr;
   const int32_t* nbr = A.nbr;
   const float inv_edge = A.inv_edge;
-  const auto div = [inv_edge](uint32_t x) { return hea_cell_div_small(x, inv_edge); };
+  int seq = 0;
+  auto post = [&](const int4& v) {
+    ++seq;
+    if (lane == 0) {
+      *reinterpret_cast<int4*>(T.vec + kCmd) = v;
+      __hip_atomic_store(T.vec + kCmdSeq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+  };
   // lane (s, h, x) takes entry (a, x) (h = 0) or (b, x) of an accepted swap
   // (lanes beyond them repeat an entry: they write the same values).  Taken
   // anew where it is used: kept over the rounds, what follows from it spills.
@@ -253,46 +365,19 @@ __device__ __forceinline__ void guided_service(const HeaMcArgs& A, const GuidedT
   double beta = 0.0;
   __builtin_amdgcn_s_setprio(3);
 
+  // The fitness after a swap that the window decided (lane 0).  Of a round's
+  // first one only behind a barrier: the other waves' decide() reads the old.
+  auto estimate = [&](const Decision& d) {
+    sh->pfm = 2;
+    sh->fest = sh->fest + d.xmin;
+  };
   // Accept of swap (s1: a -> b, s2: b -> a): exact rows, tables, species,
   // records and the round's maps.
   auto apply = [&](const Decision& d, const Winner<PT>& win, bool first) {
-    // items lane and lane + 64 of [0, 2 Z): a neighbour of s1, then of s2
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int t = opaque(lane) + 64 * u;
-      const bool one = t < Zs, on = t < 2 * Zs;
-      const int vec = T.vec[on ? (one ? t : t - Zs) : 0];
-      const HeaCellSite c = hea_cell_site<LT>(one ? d.s1 : d.s2, L, div);
-      int id = 0;
-#pragma unroll
-      for (int x = 0; x < 3; ++x) {
-        int V = 2 * c.c[x] + c.p[x] + ((vec >> (3 * x)) & 7) - 2;
-        V = V < 0 ? V + 2 * L : V >= 2 * L ? V - 2 * L : V;
-        using ST = HeaShells<LT>;
-        const int Bx = ST::BCC ? (x == 2) : x;
-        const int Ax = x == 0 ? ST::NB * L * L : x == 1 ? ST::NB * L : ST::NB;
-        id += hea_mul24(Ax, V >> 1) + Bx * (V & 1);
-      }
-      const int s = vec >> 9;
-      const int os = s == 0 ? RecBits<LT>::o(0) : s == 1 ? RecBits<LT>::o(1) : RecBits<LT>::o(2);
-      // the last species has no field (its count is implied)
-      const unsigned long long fa = d.a < K - 1 ? 1ull << (d.a * RecBits<LT>::W + os) : 0ull;
-      const unsigned long long fb = d.b < K - 1 ? 1ull << (d.b * RecBits<LT>::W + os) : 0ull;
-      const unsigned long long dv = one ? fb - fa : fa - fb;  // modulo 2^64
-      if (on) {
-        if constexpr (RL)
-          atomicAdd(rec + id, dv);
-        else
-          __hip_atomic_fetch_add(rec + id, dv, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        const uint32_t mb = cmap_bit(id);
-        atomicOr(&T.cmap[mb >> 5], 1u << (mb & 31u));
-        if (!RL) atomicOr(&T.bmap[(uint32_t)id >> (blk + 5)], 1u << (((uint32_t)id >> blk) & 31u));
-      }
-    }
-    if (lane < 2) {
-      const uint32_t mb = cmap_bit(lane == 0 ? d.s1 : d.s2);
-      atomicOr(&T.cmap[mb >> 5], 1u << (mb & 31u));
-    }
+    if (help)
+      post(make_int4(d.s1, d.s2, d.a, d.b));
+    else
+      touch<KMAX, LT, RL>(T, rec, make_int4(d.s1, d.s2, d.a, d.b), L, blk, inv_edge, lane);
     const Entry en = entry_of(lane);
     const int sv_s = en.s, sv_h = en.h, sv_x = en.x;
     const int r = sv_h ? d.b : d.a;
@@ -324,10 +409,7 @@ __device__ __forceinline__ void guided_service(const HeaMcArgs& A, const GuidedT
     if (lane == 0) {
       T.sp.set(d.s1, d.b);
       T.sp.set(d.s2, d.a);
-      if (d.kind == 2) {
-        sh->pfm = 2;
-        sh->fest = sh->fest + d.xmin;
-      }
+      if (d.kind == 2 && !first) estimate(d);
       sh->gmax = first ? __float_as_uint(top) : max(sh->gmax, __float_as_uint(top));
     }
     wave_sync();
@@ -368,6 +450,8 @@ __device__ __forceinline__ void guided_service(const HeaMcArgs& A, const GuidedT
       apply(d, win, true);
       if (multi > 1) {
         __syncthreads();  // BS
+        if (d.kind == 2 && lane == 0) estimate(d);
+        wave_sync();
         int j, c12[S], a, b;
         int2 pr;
         PT MA[S], MB[S];
@@ -387,6 +471,7 @@ __device__ __forceinline__ void guided_service(const HeaMcArgs& A, const GuidedT
         };
         load();
         for (int step = 1; step < multi; ++step) {
+          if (help) await(T.vec + kCmdDone, seq);
           if (j >= 0) {  // a touched proposal's walk is stale: dropped for good
             const uint32_t b1 = cmap_bit(pr.x), b2 = cmap_bit(pr.y);
             if (((T.cmap[b1 >> 5] >> (b1 & 31u)) | (T.cmap[b2 >> 5] >> (b2 & 31u))) & 1u) j = -1;
@@ -444,10 +529,15 @@ __device__ __forceinline__ void guided_service(const HeaMcArgs& A, const GuidedT
           }
           apply(d, win, false);
         }
+        if (help) {  // (a command is never replaced before it was answered)
+          await(T.vec + kCmdDone, seq);
+          post(make_int4(-1, 0, 0, 0));
+        }
       }
       if (lane < HEA_MAX_S) sh->vb[lane] = 0ull;  // the workers take the new bounds
     }
     __syncthreads();  // BA
+    if (multi <= 1 && d.kind == 2 && lane == 0) estimate(d);
     if (hit && lane == 0 && A.first_hit)
       atomicMin(A.first_hit, (unsigned long long)wall_clock64());
     hit = false;
@@ -742,7 +832,7 @@ __global__ __launch_bounds__(kMaxSearchThreads, 3) void k_guided(HeaMcArgs A) {
   const HeaConst& P = *A.pc;
   const int l = blockIdx.x, nthr = blockDim.x, tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int nw = (nthr >> 6) - 1;  // worker waves
+  const int nw = (A.task + 63) >> 6;  // worker waves; then the service wave and the helper
   const int N = A.N;
 
   GuidedTab<KMAX, RL> T;
@@ -754,6 +844,7 @@ __global__ __launch_bounds__(kMaxSearchThreads, 3) void k_guided(HeaMcArgs A) {
   for (int e = tid; e < HEA_MAX_S * KMAX * SearchLayout<KMAX>::KP; e += nthr)
     T.UV[e] = make_double2(0.0, 0.0);
   if (tid < 64) T.sl[tid] = -1;
+  if (tid >= kCmdSeq && tid < 64) T.vec[tid] = 0;
   if (tid < HEA_MAX_S) {
     sh->args.delta[tid] = P.delta[tid];
     sh->args.weight[tid] = P.weight[tid];
@@ -827,9 +918,11 @@ __global__ __launch_bounds__(kMaxSearchThreads, 3) void k_guided(HeaMcArgs A) {
   __syncthreads();
 
   if (wave == nw)
-    guided_service<KMAX, LT, RL>(A, T, rec, l, nw, lane);
+    guided_service<KMAX, LT, RL>(A, T, rec, l, nw, nthr > 64 * (nw + 1), lane);
+  else if (wave > nw)
+    guided_helper<KMAX, LT, RL>(A, T, rec, nw, lane);
   else
-    guided_worker<KMAX, LT, RL>(A, T, rec, l, nw, wave, tid, nthr - 64);
+    guided_worker<KMAX, LT, RL>(A, T, rec, l, nw, wave, tid, nw * 64);
 
   if (tid == 0) {
     double f = sh->pf;
@@ -896,7 +989,12 @@ HeaSearchPlan hea_guided_plan(const HeaConst& c, int lt, int task, int blk, int 
     p.lds = guided_lds(c.K, task, c.N, blk, false);
   }
   if ((int64_t)p.lds > max_lds) return HeaSearchPlan();
-  p.threads = ((task + 63) & ~63) + 64;
+  // A helper wave where it costs no resident workgroup: three waves a SIMD fit
+  // (registers), and as many workgroups as their LDS.
+  const int waves = ((task + 63) >> 6) + 1, by_lds = (int)(160 * 1024 / p.lds);
+  const bool help = waves + 1 <= kMaxSearchThreads / 64 &&
+                    std::min(12 / (waves + 1), by_lds) == std::min(12 / waves, by_lds);
+  p.threads = 64 * (waves + (help ? 1 : 0));
   return p;
 }
 
