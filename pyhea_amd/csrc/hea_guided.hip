@@ -18,6 +18,10 @@
 //     (winner_entry, refresh_fold, screen_fold): the neighbours whose records
 //     change and the adjacency come from coordinates, so no step waits for
 //     neighbour rows (only a replay reads them).
+//   * a helper wave updates the records and maps of the swap's neighbours (84 on
+//     FCC) while the service wave forms the rows and tables: 256 lattices of
+//     108000 sites 62.3 -> 56.7 ms, 4000 sites 7.80 -> 7.21 ms.  (That it also
+//     screens a shell of the shortlist gained nothing.)
 //   * meanwhile the workers draw the next round's candidates (they depend on
 //     the stream alone) and fetch their records.  A candidate's records are
 //     read one lane at a time, one line per request, and that would bound the
@@ -989,7 +993,8 @@ HeaSearchPlan hea_guided_plan(const HeaConst& c, int lt, int task, int blk, int 
     p.lds = guided_lds(c.K, task, c.N, blk, false);
   }
   if ((int64_t)p.lds > max_lds) return HeaSearchPlan();
-  // A helper wave where it costs no resident workgroup: three waves a SIMD fit
+  // A helper wave (8 to 10 % of a search, see above) where it costs no resident
+  // workgroup, which would cost far more on a full chip: three waves a SIMD fit
   // (registers), and as many workgroups as their LDS.
   const int waves = ((task + 63) >> 6) + 1, by_lds = (int)(160 * 1024 / p.lds);
   const bool help = waves + 1 <= kMaxSearchThreads / 64 &&

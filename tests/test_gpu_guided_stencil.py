@@ -59,3 +59,12 @@ def test_equimolar_replays(gpu, monkeypatch, counts):
     spec = make_problem("FCC", 4, None, counts=counts, target_seed=2)
     spec.target[:] = 0.0
     _same(monkeypatch, spec, 4, 256, 6, 12, 8, iters=2)
+
+
+@pytest.mark.parametrize("task", [192, 256, 449, 640, 641])
+@pytest.mark.parametrize("accepts", [1, 2, 8])
+def test_with_and_without_the_helper_wave(gpu, monkeypatch, task, accepts):
+    """Workgroups of 4 to 12 waves, of which those that lose no residency have
+    the wave that updates the records."""
+    spec = make_problem("BCC", 12, [4, 3, 2, 1], target_seed=6)
+    _same(monkeypatch, spec, 3, task, 3, 6, accepts)
