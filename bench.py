@@ -50,7 +50,7 @@ def bytes_per_eval(sum_z: int) -> int:
     return 2 * sum_z * (4 + 1) + 2
 
 
-def profiled_traffic(workload: str, kernel: str = "k_local_mc", key: str = "traffic_bytes_per_launch",
+def profiled_traffic(workload: str, kernel: str = "k_search", key: str = "traffic_bytes_per_launch",
                      fname: str | None = None):
     """HBM bytes per launch (or per step) from the committed rocprofv3 byte
     counters (FETCH_SIZE and WRITE_SIZE, scaled by a copy kernel of known
@@ -326,11 +326,12 @@ def time_to_fitness(a):
         "plain": plain,
         "roofline": {"bound": "hbm", "achieved": round(ach, 1), "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": round(ach / HBM_PEAK_GBS, 4),
-                     "traffic": (profiled_traffic("guided-fcc30", "k_local_mc")
+                     "traffic": (profiled_traffic("", fname="k_guided_fcc30.md")
                                  if a.workload == "ttf-fcc30" else
                                  profiled_traffic("", key="guided_traffic_bytes_per_launch",
                                                   fname="k_local_mc_fcc50.md")),
-                     "kernel": "k_local_mc (guided, batch of one problem)",
+                     "kernel": ("k_guided" if a.workload == "ttf-fcc30" else
+                                "k_local_mc") + " (guided, batch of one problem)",
                      "launches": len(launches),
                      "avg_launch_ms": round(float(ms.mean()), 3),
                      "bytes_per_launch": int(byts // len(launches)),
@@ -390,8 +391,8 @@ def batched(a):
                    "converge_depth": D, "seed": seed, "grid": shape["grid"], "tile": shape["tile"]},
         "roofline": {"bound": "hbm", "achieved": round(byts / dt / 1e9, 1), "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": round(byts / dt / 1e9 / HBM_PEAK_GBS, 4),
-                     "traffic": profiled_traffic(a.workload, "k_local_mc_batch"),
-                     "kernel": "k_local_mc_batch (whole iterations)"},
+                     "traffic": profiled_traffic(a.workload, "k_search_batch"),
+                     "kernel": "k_search_batch (whole iterations)"},
     }
     print(json.dumps(out))
 
@@ -601,7 +602,7 @@ def main():
         "unit": "GB/s",
         "frac": round(achieved / HBM_PEAK_GBS, 4),
         "traffic": profiled_traffic(a.workload),
-        "kernel": "k_local_mc",
+        "kernel": "k_search",
         "bytes_per_eval": bpe,
         "avg_launch_ms": round(float(ms.mean()), 4),
         "evals_per_launch": int(ev.sum() // n_launch),

@@ -119,7 +119,11 @@ int hea_local_mc(hea_problem p, int32_t solutions, uint8_t* lattices, double* fi
  * and solution (8 * solutions * N bytes) for its walk; hea_local_mc and
  * hea_local_mc_device grow the problem's buffer for it on demand, sessions
  * and batches allocate theirs when created (or when a tile or guide call
- * changes the placement).  Results are the same with or without it. */
+ * changes the placement).  Results are the same with or without it.  Tables
+ * that are an FCC or BCC supercell's translation stencil (cell edge 3 to 255, ids
+ * cell by cell; rows in any order) are recognised when the problem is created:
+ * their plain search keeps the species in LDS up to about 130000 sites, and two
+ * species a byte up to about 270000. */
 int hea_local_mc_device(hea_problem p, int32_t solutions, void* d_lattices, void* d_fitness,
                         int32_t parallel_task, int32_t converge_depth, uint64_t seed,
                         uint32_t iter, uint32_t phase, void* stream);
@@ -173,7 +177,9 @@ int hea_session_init(hea_session s);
  * reference: `tile` proposal slots per pass (64, 128, 192 or 256).  A shell
  * whose neighbour list is at least twice as long as the others' is walked by
  * 2 or 4 lanes per slot (at most 1024 lanes).  Results do not depend on it;
- * the autotuner (pyhea_amd/autotune.py) picks it. */
+ * the autotuner (pyhea_amd/autotune.py) picks it.  On stencil lattices with at
+ * most 704 proposals a round the search takes the whole round in one pass
+ * whatever the tile. */
 int hea_session_tile(hea_session s, int32_t tile);
 /* Guided proposals, no counterpart in the reference.  The local search keeps
  * every site's neighbour species counts and the gradient of the fitness
@@ -226,7 +232,9 @@ int hea_session_destroy(hea_session s);
 /* Batched search with no counterpart in the reference (which runs one
  * problem per call, accelerate.cpp:713-763): n_probs independent problems on
  * one device, each with its own population of `solutions` lattices, all
- * searched by one persistent local-search launch per phase.  Problem p
+ * searched by one local-search launch per phase (stencil lattices whose species
+ * fit in LDS longest first, one workgroup a lattice; the others by a persistent
+ * launch).  Problem p
  * draws from seed `seed + p`, so its population equals
  * hea_hcs_run(probs[p], ..., seed + p, ...).  Problems must share the
  * device, the shell count and have no self neighbours; parallel_task and

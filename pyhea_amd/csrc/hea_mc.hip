@@ -1,4 +1,8 @@
-// Greedy best-of-T local search (the hot path), one workgroup per lattice.
+// Greedy best-of-T local search, one workgroup per lattice: the general kernel.
+// FCC and BCC supercells whose table is the translation stencil take the kernels
+// of hea_search.h (plain) and hea_guided.hip instead, where their limits allow; this
+// one takes every other table, rounds beyond 704 proposals, species in HBM, and
+// batches of several guided problems.
 //
 // Semantics follow pyhea/cpp/accelerate.cpp:601-694 (local_parallel_monte_carlo)
 // and :498-570 (calculate_fitness_incremental):
