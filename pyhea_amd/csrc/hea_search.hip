@@ -9,16 +9,20 @@ namespace {
 
 // One population each of many problems: workgroup i searches lattice
 // items[i].y of problem items[i].x, longest first.  One launch for all of them,
-// so that the tail of a phase is made of short searches; table widths 4, 6 and
-// 8 (absent species hold zeros) keep the instantiations few.
+// so that the tail of a phase is made of short searches.  Every species count has
+// tables of its own width: padded to 4, 6 and 8 species an odd count paid a fifth
+// more screen (uneven problems of 3 to 6 species: 61.3 -> 57.9 ms).
 template <int LT>
 __device__ __forceinline__ void search_item(const HeaMcArgs& A, int l, unsigned char* smem) {
-  if (A.K <= 4)
-    search_lattice<4, false, LT, false>(A, l, smem);
-  else if (A.K <= 6)
-    search_lattice<6, false, LT, false>(A, l, smem);
-  else
-    search_lattice<8, false, LT, false>(A, l, smem);
+  switch (A.K) {
+    case 2: return search_lattice<2, true, LT, false>(A, l, smem);
+    case 3: return search_lattice<3, true, LT, false>(A, l, smem);
+    case 4: return search_lattice<4, true, LT, false>(A, l, smem);
+    case 5: return search_lattice<5, true, LT, false>(A, l, smem);
+    case 6: return search_lattice<6, true, LT, false>(A, l, smem);
+    case 8: return search_lattice<8, true, LT, false>(A, l, smem);
+    default: return search_lattice<8, false, LT, false>(A, l, smem);
+  }
 }
 
 __global__ __launch_bounds__(kMaxSearchThreads, 4) void k_search_batch(
@@ -50,10 +54,9 @@ size_t search_lds(int K, int task, size_t n) {
 HeaSearchPlan hea_search_plan(const HeaConst& c, int lt, int task, int64_t max_lds, bool batch) {
   HeaSearchPlan p;
   if (lt == HEA_LT_NONE || task > kMaxSearchThreads - 64) return p;
-  const int width = batch ? (c.K <= 4 ? 4 : c.K <= 6 ? 6 : 8) : c.K;
-  size_t lds = search_lds(width, task, Species<false, 5>::bytes(c.N));
+  size_t lds = search_lds(c.K, task, Species<false, 5>::bytes(c.N));
   if ((int64_t)lds > max_lds && !batch) {  // two species a byte
-    lds = search_lds(width, task, Species<true, 5>::bytes(c.N));
+    lds = search_lds(c.K, task, Species<true, 5>::bytes(c.N));
     p.nib = true;
   }
   if ((int64_t)lds > max_lds) return HeaSearchPlan();

@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 
 from oracle import Oracle
-from pyhea_amd.hcs import Problem
+from pyhea_amd.hcs import Batch, Problem
 from pyhea_amd.problem import ProblemSpec, make_problem
 
 pytestmark = pytest.mark.gpu
@@ -92,3 +92,18 @@ def test_two_species_a_byte_equals_the_hbm_walk(gpu, monkeypatch, latt, edge, sh
 def test_walks_by_cell(gpu, edge, shells, k):
     """Each parity of the edge and each width of the histograms."""
     _check(make_problem("FCC", edge, np.arange(2, k + 2), shells=shells, target_seed=k), 100, 3)
+
+
+def test_batch_of_every_species_count(gpu):
+    """One problem per table width in one launch, against its own search."""
+    specs = [make_problem("FCC" if k % 2 else "BCC", 4, np.arange(2, k + 2), target_seed=k)
+             for k in range(2, 9)]
+    probs = [Problem.from_spec(s) for s in specs]
+    b = Batch(probs, 5, 96, 3, seed=40)
+    b.init()
+    b.step(2)
+    for q, p in enumerate(probs):
+        lat, fit, st = b.read(q)
+        lo, fo, so = p.run_hcs(5, 2, 96, 3, seed=40 + q)
+        assert np.array_equal(lat, lo) and np.array_equal(_bits(fit), _bits(fo))
+        assert st["accepts"] == so["accepts"]
