@@ -35,7 +35,8 @@
 // What bounds it: the accepts, half of a round's 65000 cycles at 108000 sites (one
 // wave's latency; 5000 each), then the candidates' records (a third).  256 lattices
 // of 108000 sites, 512 slots, 12 candidates, up to 8 accepts: 57.9 ms a launch, 148.3
-// with k_local_mc; 128 of 4000 sites, 256 slots: 12.7 ms a search, 36.5.
+// with k_local_mc; 128 of 4000 sites, 256 slots, a session of two iterations: 12.7
+// ms, 36.5.
 //
 // Barriers of a round: BD difference table ready; B1 minima published; BS
 // shortlist ready (accepts only); BA accepts done.

@@ -35,10 +35,10 @@
 // What bounds it: LDS (40 to 51 % of a CU's cycles, a third of them bank
 // conflicts) and vector issue (61 %), in a chain of dependent steps; of a round of
 // 10000 to 13500 cycles the walk is a third, the screen a fifth, drawing and
-// listing the proposals a quarter.  Local search I on a random population, one
-// draw each, against k_local_mc: 512 lattices of 8192 sites, 256 proposals, 5.2 ms,
-// 11.2; 256 of 108000 sites, 512 proposals, 99.5 ms, 216; 64 of 256000 sites, two
-// species a byte, 2.1 times as fast as the walk through HBM.
+// listing the proposals a quarter.  Launches on average of a session's searches,
+// against k_local_mc: 512 lattices of 8192 sites, 256 proposals, 3.67 ms, 7.47; 256
+// of 108000 sites, 512 proposals, 50.7 ms, 155.0; 64 of 256000 sites, two species a
+// byte, 2.1 times as fast as the walk through HBM.
 #pragma once
 #include "hea_exact.h"
 #include "hea_internal.h"

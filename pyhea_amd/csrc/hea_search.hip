@@ -53,8 +53,8 @@ size_t search_lds(int K, int task, size_t n) {
 
 // Stencil lattices take this search up to 704 proposals (eleven worker waves, the
 // most whose registers and the service wave's fit a workgroup), bytes where they
-// fit, else two species a byte; both are two to three times as fast as k_local_mc
-// at every size measured (108 to 270000 sites), bytes a tenth faster than nibbles.
+// fit (a nibble costs two instructions more per neighbour), else two species a byte:
+// 1.5 to 3 times as fast as k_local_mc at every size measured, 108 to 270000 sites.
 HeaSearchPlan hea_search_plan(const HeaConst& c, int lt, int task, int64_t max_lds, bool batch) {
   HeaSearchPlan p;
   if (lt == HEA_LT_NONE || task > kMaxSearchThreads - 64) return p;
